@@ -3,6 +3,8 @@
 #include <math.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace noise {
@@ -50,16 +52,19 @@ __global__ __launch_bounds__(1024) void fitness_kernel(const float* __restrict__
   }
 }
 
-// grad[o, i] = scale sum_j w_j a_j[o] b_j[i] (eggroll.py:159-161: (w a)^T b over the pairs), on fp32 MFMA
-// (v_mfma_f32_32x32x2_f32, full fp32 products and sums). A workgroup owns a 128 x 128 output tile, each of its 4 waves
-// 64 x 64 (2 x 2 MFMA tiles); the pairs stream through two LDS stages of 16: a_j[o0 .. o0+127] and w_j b_j[i0 ..]
-// as rows [pair][128] padded to 160 floats, so the two pair rows of one operand read (lanes 0..31 and 32..63) fall
-// in opposite halves of the 64 banks. Every load is a 256-byte row segment (thread: one column, 8 of the 16 rows);
-// columns past out / in and pairs past the last read as zeros, so offsets and sizes need no alignment.
-// One launch covers a list of matrices (jobs, by value in the kernel arguments): the launch's tiles are numbered job by
-// job, each job's in row-major order over ceil(out / 128) x ceil(in / 128); tile t belongs to the job whose range
-// [tile0, next tile0) holds it, and each XCD takes a contiguous run of tile numbers.
-constexpr int kOgTile = 128, kOgK = 16, kOgPitch = 160, kOgMaxJobs = 64;
+// ---- sums of outer products -------------------------------------------------------------------------------------
+// Two kernels over a list of matrices (jobs, by value in the kernel arguments). A launch's tiles are numbered job by
+// job, each job's in row-major order; tile t belongs to the job whose range [tile0, next tile0) holds it, and each XCD
+// takes a contiguous run of tile numbers.
+//
+// In both a wave reads its MFMA operands straight from memory in the MFMA layout (a load is two 128-byte row
+// segments): the rows k of a and b already have the output's columns side by side, so there is no LDS staging, no
+// barrier and no transpose, and a step's loads are issued a whole step ahead of the MFMAs that take them. (Staging
+// 128 x 128 tiles in LDS with one 4-byte load and store per value ran at 41 TFLOP/s.) Loads go through buffer
+// resources that end with the step's last live value: rows past the last one read as zeros, columns past the matrix
+// feed only outputs that are not stored, so offsets and sizes need no alignment. Row strides too long for 32-bit
+// offsets take 64-bit addresses (kWide).
+constexpr int kOgMaxJobs = 64;
 
 struct OgJob {
   int64_t a_off, b_off;  // column offsets of a (out values) and b (in values) in their rows
@@ -74,104 +79,320 @@ struct OgJobs {
   OgJob job[kOgMaxJobs];
 };
 
-// Sum over k < n_k of a_k b_k^T with row k of A at a_rows + k a_stride (fp32) and of B at b_rows + k b_stride (fp32,
-// or bf16 with b_bf16), b_k scaled by weight[k] when a weight is given.
-__global__ __launch_bounds__(256) void outer_grad_kernel(const float* __restrict__ a_rows, int64_t a_stride,
-                                                         const void* __restrict__ b_rows, int64_t b_stride, int b_bf16,
-                                                         const float* __restrict__ weight, int64_t pairs, float scale,
-                                                         OgJobs jobs) {
-  __shared__ float as[2][kOgK][kOgPitch];
-  __shared__ float bs[2][kOgK][kOgPitch];
-  // Workgroups are dispatched round-robin over the 8 XCDs; XCD x takes the contiguous tile range
-  // [x per, (x + 1) per), so the tiles of one matrix, which read the same a and b slices, share one L2.
+// The workgroup's tile number (or -1 past the last: the grid's round-up) and its job. Workgroups are dispatched
+// round-robin over the 8 XCDs; XCD x takes the contiguous tile range [x per, (x + 1) per), so the tiles of one matrix,
+// which read the same a and b slices, share one L2.
+__device__ __forceinline__ int og_tile(const OgJobs& jobs, int* job) {
   const int per = (int)(gridDim.x / 8);
-  const int tid_ = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-  if (tid_ >= jobs.total) return;  // the grid's round-up
+  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (t >= jobs.total) return -1;
   int jb = 0;
-  while (jb + 1 < jobs.n && tid_ >= jobs.job[jb + 1].tile0) ++jb;
-  const OgJob& job = jobs.job[jb];
-  const int64_t a_off = job.a_off, b_off = job.b_off, out = job.out, in = job.in;
-  float* __restrict__ grad = job.grad;
-  const int tile = tid_ - job.tile0;
-  const int64_t o0 = (int64_t)(tile / job.n_in_tiles) * kOgTile, i0 = (int64_t)(tile % job.n_in_tiles) * kOgTile;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wo = (wave >> 1) * 64, wi = (wave & 1) * 64;
-  const int col = tid & 127, row0 = tid >> 7;  // loader: column col of rows row0, row0 + 2, ..., row0 + 14
-  const bool a_in = o0 + col < out, b_in = i0 + col < in;
+  while (jb + 1 < jobs.n && t >= jobs.job[jb + 1].tile0) ++jb;
+  *job = jb;
+  return t - jobs.job[jb].tile0;
+}
 
-  float ra[8], rb[8];
-  auto load = [&](int64_t j0) {
+// One wave's operand values of a step of 16 rows: T column tiles of 32, lane l column l % 32, value e of lane half
+// h = l / 32 row 2 e + h (kPair, the k order of 8 fp32 MFMAs) or 8 h + e (of one bf16 MFMA).
+template <int T, bool kPair, bool kBf16, bool kWide>
+struct OgOperand {
+  const char* base;  // row 0, the wave's first column
+  int64_t stride;    // bytes
+  int width;         // columns from there on
+  int vo[kWide ? 1 : 8];
+  typedef float Values[T][8];
+  static constexpr int kElt = kBf16 ? 2 : 4;
+  __device__ __forceinline__ static int row(int half, int e) { return kPair ? 2 * e + half : 8 * half + e; }
+  __device__ __forceinline__ OgOperand(const void* rows, int64_t ld, int64_t col0, int width_, int lane)
+      : base((const char*)rows + col0 * kElt), stride(ld * kElt), width(width_) {
+    if constexpr (!kWide) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int64_t j = j0 + row0 + 2 * q;
-      const bool live = j < pairs;
-      const int64_t jj = live ? j : 0;
-      ra[q] = (live && a_in) ? a_rows[jj * a_stride + a_off + o0 + col] : 0.f;
-      float bv = 0.f;
-      if (live && b_in) {
-        const int64_t at = jj * b_stride + b_off + i0 + col;
-        bv = b_bf16 ? bf16_to_f32(((const bf16_t*)b_rows)[at]) : ((const float*)b_rows)[at];
-        if (weight) bv = weight[j] * bv;
-      }
-      rb[q] = bv;
+      for (int e = 0; e < 8; ++e) vo[e] = row(lane >> 5, e) * (int)stride + (lane & 31) * kElt;
     }
-  };
-  auto store = [&](int st) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      as[st][row0 + 2 * q][col] = ra[q];
-      bs[st][row0 + 2 * q][col] = rb[q];
-    }
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int v = 0; v < 2; ++v)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
-
-  load(0);
-  store(0);
-  __syncthreads();
-  const int64_t n_steps = (pairs + kOgK - 1) / kOgK;
-  const int kr = lane >> 5, lc = lane & 31;  // operand lane: pair row kr of the k pair, column lc of the 32
-  for (int64_t t = 0; t < n_steps; ++t) {
-    const int st = (int)(t & 1);
-    const bool more = t + 1 < n_steps;
-    if (more) load((t + 1) * kOgK);
-#pragma unroll
-    for (int s = 0; s < kOgK / 2; ++s) {
-      float fa[2], fb[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        fa[u] = as[st][2 * s + kr][wo + 32 * u + lc];
-        fb[u] = bs[st][2 * s + kr][wi + 32 * u + lc];
-      }
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int v = 0; v < 2; ++v) acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u], fb[v], acc[u][v], 0, 0, 0);
-    }
-    if (more) store(st ^ 1);
-    __syncthreads();
   }
-
-  // accumulator register r of tile (u, v): row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
+  // v = rows k0 .. k0 + live - 1, 1 <= live <= 16
+  __device__ __forceinline__ void load(int64_t k0, int live, int lane, Values& v) const {
+    if constexpr (kWide) {
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+      for (int e = 0; e < 8; ++e) {
+        const int k = row(lane >> 5, e);
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t o = o0 + wo + 32 * u + 8 * (r >> 2) + 4 * kr + (r & 3), i = i0 + wi + 32 * v + lc;
-        if (o < out && i < in) {
-          float* gp = grad + o * in + i;
-          *gp = jobs.accumulate ? fmaf(scale, acc[u][v][r], *gp) : scale * acc[u][v][r];
+        for (int t = 0; t < T; ++t) {
+          const int c = 32 * t + (lane & 31);
+          const char* at = base + (k0 + k) * stride + (int64_t)c * kElt;
+          const bool ok = k < live && c < width;
+          if constexpr (kBf16) v[t][e] = __uint_as_float(ok ? *(const bf16_t*)at : 0u);
+          else v[t][e] = ok ? *(const float*)at : 0.f;
         }
       }
+    } else {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(base + k0 * stride), 0, (live - 1) * (int)stride + width * kElt, 0x00020000);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int at = vo[e] + 32 * kElt * t;
+          if constexpr (kBf16) v[t][e] = __uint_as_float((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at, 0, 0));
+          else v[t][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0));
+        }
+    }
+  }
+};
+
+// Steps k0, k0 + kStride, ... < n on two register sets: the next step's loads are issued before this step's arithmetic.
+template <class Step, int kStride, class Load, class Multiply>
+__device__ __forceinline__ void og_pipeline(int64_t k0, int64_t n, const Load& load, const Multiply& multiply) {
+  if (k0 >= n) return;
+  Step s0, s1;
+  load(k0, s0);
+  while (true) {
+    const bool more1 = k0 + kStride < n;
+    if (more1) load(k0 + kStride, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(s0);
+    if (!more1) break;
+    k0 += 2 * kStride;
+    const bool more0 = k0 < n;
+    if (more0) load(k0, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(s1);
+    if (!more0) break;
+  }
 }
+
+// accumulator register r of a 32 x 32 tile: row 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32
+__device__ __forceinline__ void og_store(const f32x16& acc, int o0, int i0, const OgJob& job, int accumulate, float scale,
+                                         int lane) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int64_t o = o0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), i = i0 + (lane & 31);
+    if (o < job.out && i < job.in) {
+      float* gp = job.grad + o * job.in + i;
+      *gp = accumulate ? fmaf(scale, acc[r], *gp) : scale * acc[r];
+    }
+  }
+}
+
+// grad[o, i] = scale sum_j a_j[o] (w_j b_j[i]) (eggroll.py:159-161: (w a)^T b over the pairs) on fp32 MFMA
+// (v_mfma_f32_32x32x2_f32: fp32 products and sums, the pairs in order). A wave owns TM x TM tiles of 32 x 32, four
+// waves 2 x 2 of those. Bound by the MFMA issue at 2 x 2 (32 MFMAs of 64 cycles per 16 pairs against 40 loads and 16
+// multiplications).
+template <int TM, bool kWide>
+__global__ __launch_bounds__(256, TM == 2 ? 3 : 4) void outer_grad_kernel(const float* __restrict__ rows, int64_t stride,
+                                                                          const float* __restrict__ weight,
+                                                                          int64_t pairs, float scale, OgJobs jobs) {
+  int jb;
+  const int tile = og_tile(jobs, &jb);
+  if (tile < 0) return;
+  const OgJob& job = jobs.job[jb];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o0 = (tile / job.n_in_tiles) * 64 * TM + (wave >> 1) * 32 * TM;
+  const int i0 = (tile % job.n_in_tiles) * 64 * TM + (wave & 1) * 32 * TM;
+  if (o0 >= job.out || i0 >= job.in) return;  // a wave past the matrix (there is no barrier)
+  OgOperand<TM, true, false, kWide> a(rows, stride, job.a_off + o0, job.out - o0, lane);
+  OgOperand<TM, true, false, kWide> b(rows, stride, job.b_off + i0, job.in - i0, lane);
+  f32x16 acc[TM][TM];
+#pragma unroll
+  for (int u = 0; u < TM; ++u)
+#pragma unroll
+    for (int v = 0; v < TM; ++v) acc[u][v] = f32x16{};
+  float ra[TM][8], rb[TM][8], w[8];
+  auto load = [&](int64_t k0) {
+    const int live = (int)(pairs - k0 < 16 ? pairs - k0 : 16);
+    a.load(k0, live, lane, ra);
+    b.load(k0, live, lane, rb);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(weight + k0), 0, live * 4, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      w[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, 4 * (lane >> 5) + 8 * e, 0, 0));
+  };
+  // One register set and three waves per SIMD: a step's values are taken (and weighted), then the next step's loads go
+  // out ahead of the MFMAs. 690 us for the 8-block model's 2,304 tiles at 1,024 pairs (112 TFLOP/s); two register sets
+  // at two waves per SIMD 800 us.
+  load(0);
+  for (int64_t k0 = 0; k0 < pairs; k0 += 16) {
+    float av[TM][8], bv[TM][8];
+#pragma unroll
+    for (int u = 0; u < TM; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        av[u][e] = ra[u][e];
+        bv[u][e] = w[e] * rb[u][e];
+      }
+    if (k0 + 16 < pairs) load(k0 + 16);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int v = 0; v < TM; ++v)
+          acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u][e], bv[v][e], acc[u][v], 0, 0, 0);
+  }
+#pragma unroll
+  for (int u = 0; u < TM; ++u)
+#pragma unroll
+    for (int v = 0; v < TM; ++v) og_store(acc[u][v], o0 + 32 * u, i0 + 32 * v, job, jobs.accumulate, scale, lane);
+}
+
+// grad[o, i] = scale sum_t error[t, o] x[t, i] with fp32 products on the bf16 matrix units. An fp32 operand is split
+// into three bf16 parts x = x1 + x2 + x3, each the rounded rest of the one before, which hold its 24 bits; of the nine
+// products of two such operands the six of the leading orders are summed in fp32, smallest first. What is left out is
+// below 2^-25 of a product, less than the rounding of an fp32 multiply, and an accumulator rounds 6 times per 16 rows
+// where v_mfma_f32_32x32x2_f32 rounds 8 times. Six v_mfma_f32_32x32x16_bf16 take 192 cycles per 32 x 32 x 16 block,
+// the fp32 MFMAs 512; a bf16 operand is exact in one part, so it takes three.
+//
+// A call has one matrix, often smaller than the GPU (512 x 512 outputs are 16 tiles of 128 x 128, and 16,384 rows ran
+// in 2.0 ms on those 16 workgroups), so the WK waves of a workgroup split the rows of one tile of 32 TM x 32 TM into
+// interleaved runs of 16-row steps; a fixed-order tree through LDS adds their sums (deterministic).
+// x1, x2, x3 of 8 values as MFMA fragments. An infinity, or a value that rounds to one, has the rest inf - inf, so it
+// gives NaN: the kernel repeats a tile that came out NaN on the fp32 MFMA, which has no such limits.
+struct OgSplit {
+  u32x4 p[3];
+};
+__device__ __forceinline__ OgSplit og_split(const float (&x)[8]) {
+  OgSplit s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float r0 = x[2 * j], r1 = x[2 * j + 1];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const uint32_t b = pack_bf16x2(r0, r1);
+      s.p[q][j] = b;
+      r0 -= bf16_lo(b);
+      r1 -= bf16_hi(b);
+    }
+  }
+  return s;
+}
+
+template <int TM, int WK, bool kBf16, bool kWide>
+__global__ __launch_bounds__(64 * WK, TM == 1 ? 4 : 2) void reassemble_kernel(const float* __restrict__ error,
+                                                                              int64_t error_ld,
+                                                                              const void* __restrict__ x, int64_t x_ld,
+                                                                              int64_t tokens, float scale, OgJobs jobs) {
+  __shared__ float red[WK / 2][TM * TM * 1024];
+  int jb;
+  const int tile = og_tile(jobs, &jb);
+  if (tile < 0) return;
+  const OgJob& job = jobs.job[jb];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o0 = (tile / job.n_in_tiles) * 32 * TM, i0 = (tile % job.n_in_tiles) * 32 * TM;
+  OgOperand<TM, false, false, kWide> a(error, error_ld, o0, job.out - o0, lane);
+  OgOperand<TM, false, kBf16, kWide> b(x, x_ld, i0, job.in - i0, lane);
+  f32x16 acc[TM][TM];
+#pragma unroll
+  for (int u = 0; u < TM; ++u)
+#pragma unroll
+    for (int v = 0; v < TM; ++v) acc[u][v] = f32x16{};
+  struct Step {
+    float a[TM][8], b[TM][8];
+  };
+  auto load = [&](int64_t k0, Step& st) {
+    const int live = (int)(tokens - k0 < 16 ? tokens - k0 : 16);
+    a.load(k0, live, lane, st.a);
+    b.load(k0, live, lane, st.b);
+  };
+  auto multiply = [&](const Step& st) {
+    OgSplit sa[TM], sb[TM];
+#pragma unroll
+    for (int u = 0; u < TM; ++u) {
+      sa[u] = og_split(st.a[u]);
+      if constexpr (!kBf16) sb[u] = og_split(st.b[u]);
+    }
+    if constexpr (kBf16) {
+#pragma unroll
+      for (int v = 0; v < TM; ++v)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          sb[v].p[0][j] = __float_as_uint(st.b[v][2 * j]) | (__float_as_uint(st.b[v][2 * j + 1]) << 16);
+    }
+    auto product = [&](int pa, int pb) {
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int v = 0; v < TM; ++v)
+          acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, sa[u].p[pa]),
+                                                              __builtin_bit_cast(bf16x8, sb[v].p[pb]), acc[u][v], 0, 0, 0);
+    };
+    product(2, 0);
+    if constexpr (!kBf16) {
+      product(0, 2);
+      product(1, 1);
+    }
+    product(1, 0);
+    if constexpr (!kBf16) product(0, 1);
+    product(0, 0);
+  };
+  og_pipeline<Step, 16 * WK>(16 * wave, tokens, load, multiply);
+  bool nan = false;
+#pragma unroll
+  for (int u = 0; u < TM; ++u)
+#pragma unroll
+    for (int v = 0; v < TM; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nan = nan || acc[u][v][r] != acc[u][v][r];
+  if (__builtin_expect(__ballot(nan) != 0, 0)) {
+#pragma unroll
+    for (int u = 0; u < TM; ++u)
+#pragma unroll
+      for (int v = 0; v < TM; ++v) acc[u][v] = f32x16{};
+    og_pipeline<Step, 16 * WK>(16 * wave, tokens, load, [&](const Step& st) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int u = 0; u < TM; ++u)
+#pragma unroll
+          for (int v = 0; v < TM; ++v) {
+            const float be = kBf16 ? __uint_as_float(__float_as_uint(st.b[v][e]) << 16) : st.b[v][e];
+            acc[u][v] = __builtin_amdgcn_mfma_f32_32x32x2f32(st.a[u][e], be, acc[u][v], 0, 0, 0);
+          }
+    });
+  }
+  // the waves' sums, pairwise: wave w adds wave w + s for s = WK / 2, ..., 1
+#pragma unroll
+  for (int s = WK / 2; s >= 1; s >>= 1) {
+    if (wave >= s && wave < 2 * s) {
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int v = 0; v < TM; ++v)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) red[wave - s][((u * TM + v) * 16 + r) * 64 + lane] = acc[u][v][r];
+    }
+    __syncthreads();
+    if (wave < s) {
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int v = 0; v < TM; ++v)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[u][v][r] += red[wave][((u * TM + v) * 16 + r) * 64 + lane];
+    }
+    __syncthreads();
+  }
+  if (wave != 0) return;
+#pragma unroll
+  for (int u = 0; u < TM; ++u)
+#pragma unroll
+    for (int v = 0; v < TM; ++v) og_store(acc[u][v], o0 + 32 * u, i0 + 32 * v, job, 0, scale, lane);
+}
+
+// Numbers the jobs' tiles of side x side outputs; returns how many there are (jobs.total, when they fit a grid).
+static int64_t og_number_tiles(OgJobs& jobs, int side) {
+  int64_t tiles = 0;
+  for (int k = 0; k < jobs.n; ++k) {
+    OgJob& g = jobs.job[k];
+    g.n_in_tiles = (int32_t)(((int64_t)g.in + side - 1) / side);
+    g.tile0 = (int32_t)tiles;
+    tiles += (int64_t)g.n_in_tiles * (((int64_t)g.out + side - 1) / side);
+  }
+  jobs.total = (int32_t)tiles;
+  return tiles;
+}
+static dim3 og_grid(int64_t tiles) { return dim3((unsigned)((tiles + 7) / 8 * 8)); }
+// Whether 16 rows of this many bytes each pass the 31-bit offsets of a buffer resource.
+static bool og_wide(int64_t row_bytes) { return row_bytes >= ((int64_t)1 << 31) / 16; }
 
 // grad[i] = scale sum_j w_j eps_j[i] (1-D parameters: eggroll.py:163). A block owns 8 consecutive elements; its 256
 // threads take the pairs j = t, t + 256, ... and a fixed-order tree in LDS adds their partial sums (deterministic).
@@ -331,21 +552,21 @@ extern "C" int noise_outer_grad_batch(const float* rows, int64_t stride, const f
     memset(&jobs, 0, sizeof(jobs));
     jobs.n = n - j0 < kOgMaxJobs ? n - j0 : kOgMaxJobs;
     jobs.accumulate = accumulate ? 1 : 0;
-    int64_t tiles = 0;
     for (int k = 0; k < jobs.n; ++k) {
       const int32_t j = j0 + k;
       OgJob& g = jobs.job[k];
       g.a_off = a_off[j]; g.b_off = b_off[j]; g.out = (int32_t)out[j]; g.in = (int32_t)in[j]; g.grad = grads[j];
-      g.n_in_tiles = (int32_t)((in[j] + kOgTile - 1) / kOgTile);
-      g.tile0 = (int32_t)tiles;
-      tiles += (int64_t)g.n_in_tiles * ((out[j] + kOgTile - 1) / kOgTile);
-      NOISE_REQUIRE(tiles <= INT32_MAX, "too many tiles");
     }
-    if (tiles == 0) continue;
+    // 64 x 64 outputs per wave, or 32 x 32 where those are fewer than the GPU's 1,024 SIMDs
+    const bool wide = og_wide(stride * 4), small = wide || og_number_tiles(jobs, 64) < 1024;
+    const int64_t tiles = og_number_tiles(jobs, small ? 64 : 128);
     NOISE_REQUIRE(tiles + 7 <= INT32_MAX, "too many tiles");
-    jobs.total = (int32_t)tiles;
-    hipLaunchKernelGGL(outer_grad_kernel, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream,
-                       rows, stride, (const void*)rows, stride, 0, weight, pairs, scale, jobs);
+    if (tiles == 0) continue;
+    const dim3 grid = og_grid(tiles);
+    const hipStream_t st = (hipStream_t)stream;
+    if (wide) outer_grad_kernel<1, true><<<grid, dim3(256), 0, st>>>(rows, stride, weight, pairs, scale, jobs);
+    else if (small) outer_grad_kernel<1, false><<<grid, dim3(256), 0, st>>>(rows, stride, weight, pairs, scale, jobs);
+    else outer_grad_kernel<2, false><<<grid, dim3(256), 0, st>>>(rows, stride, weight, pairs, scale, jobs);
     NOISE_LAUNCH_CHECK();
   }
   return NOISE_OK;
@@ -363,13 +584,23 @@ extern "C" int noise_reassemble(const float* error, int64_t error_ld, const void
   jobs.n = 1;
   OgJob& g = jobs.job[0];
   g.out = (int32_t)d_out; g.in = (int32_t)d_in; g.grad = grad;
-  g.n_in_tiles = (int32_t)((d_in + kOgTile - 1) / kOgTile);
-  const int64_t tiles = (int64_t)g.n_in_tiles * ((d_out + kOgTile - 1) / kOgTile);
+  // 64 x 64 outputs per workgroup of 8 waves where they give most CUs one, else 32 x 32 of 16 waves
+  const bool wide = og_wide(error_ld * 4) || og_wide(x_ld * (x_bf16 ? 2 : 4));
+  const bool small = wide || og_number_tiles(jobs, 64) < 192;
+  const int64_t tiles = og_number_tiles(jobs, small ? 32 : 64);
   NOISE_REQUIRE(tiles + 7 <= INT32_MAX, "too many tiles");
-  jobs.total = (int32_t)tiles;
-  NoiseTimer tm(kTimeReassemble, (hipStream_t)stream);
-  hipLaunchKernelGGL(outer_grad_kernel, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream,
-                     error, error_ld, x, x_ld, x_bf16 ? 1 : 0, (const float*)nullptr, tokens, scale, jobs);
+  const hipStream_t st = (hipStream_t)stream;
+  NoiseTimer tm(kTimeReassemble, st);
+#define NOISE_REASSEMBLE(TM, WK, BF, WIDE) \
+  reassemble_kernel<TM, WK, BF, WIDE><<<og_grid(tiles), dim3(64 * WK), 0, st>>>(error, error_ld, x, x_ld, tokens, scale, jobs)
+  if (wide) {
+    if (x_bf16) NOISE_REASSEMBLE(1, 16, true, true); else NOISE_REASSEMBLE(1, 16, false, true);
+  } else if (small) {
+    if (x_bf16) NOISE_REASSEMBLE(1, 16, true, false); else NOISE_REASSEMBLE(1, 16, false, false);
+  } else {
+    if (x_bf16) NOISE_REASSEMBLE(2, 8, true, false); else NOISE_REASSEMBLE(2, 8, false, false);
+  }
+#undef NOISE_REASSEMBLE
   NOISE_LAUNCH_CHECK();
   return NOISE_OK;
 }

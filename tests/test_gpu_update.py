@@ -107,6 +107,55 @@ def test_outer_grad_batch_over_several_launches(dev):
         assert torch.allclose(got.cpu().double(), want, rtol=1e-4, atol=1e-4), (a0, o, i)
 
 
+@pytest.mark.parametrize('tokens,out,n_in,bf16,pad', [
+    (1, 1, 1, False, 0),          # one row, one output
+    (15, 31, 33, False, 3),       # short of a 16-row step, edges of the 32-wide tiles, odd strides
+    (17, 65, 32, True, 1),        # a step and one row; bf16 at odd strides
+    (257, 512, 512, False, 0),    # 32 x 32 tiles, 16 waves over 17 steps
+    (300, 2048, 513, True, 5),    # 64 x 64 tiles, 8 waves, a ragged last column tile
+    (1000, 4096, 512, False, 0),
+    (3, 5, 7, False, 1 << 25),    # rows too far apart for 32-bit offsets
+])
+def test_reassemble_over_the_forms_it_takes(dev, tokens, out, n_in, bf16, pad):
+    """noise_reassemble at the edges of its tiles and steps, in both operand types, with rows apart. The bound is that of
+    `tokens` fp32 products summed in any order, each rounding at most 2^-24 of the sum of magnitudes."""
+    print(f'reassemble tokens={tokens} {out}x{n_in} bf16={bf16} pad={pad}', flush=True)
+    from noise_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(tokens + out)
+    error = torch.empty(tokens, out + pad, device=dev)[:, :out]
+    x = torch.empty(tokens, n_in + pad, device=dev, dtype=torch.bfloat16 if bf16 else torch.float32)[:, :n_in]
+    error.copy_(torch.randn(tokens, out, device=dev, generator=g))
+    x.copy_(torch.randn(tokens, n_in, device=dev, generator=g))
+    grad = torch.full((out, n_in), float('nan'), device=dev)
+    _lib.call('noise_reassemble', _lib.ptr(error), error.stride(0), _lib.ptr(x), int(bf16), x.stride(0), tokens, out,
+              n_in, 0.5, _lib.ptr(grad), _lib.stream(dev))
+    e, xd = error.double(), x.double()
+    want, size = 0.5 * e.t().contiguous() @ xd, 0.5 * e.abs().t().contiguous() @ xd.abs()
+    assert ((grad.double() - want).abs() <= (tokens + 2) * 2.0 ** -24 * size + 1e-37).all()
+
+
+def test_reassemble_keeps_infinities_and_the_largest_values(dev):
+    """Values that bf16 parts cannot hold alone: an infinity gives infinities (NaN against a zero), a NaN its row's NaN,
+    and the largest finite value the finite product."""
+    from noise_amd import _lib
+    g = torch.Generator().manual_seed(5)
+    error, x = torch.randn(40, 70, generator=g), torch.randn(40, 50, generator=g).abs() + 0.1
+    error[3, 10], error[7, 20], error[9, 30] = float('inf'), float('nan'), torch.finfo(torch.float32).max
+    x[:, 4] *= 1e-30
+    x[3, 6] = 0.0
+    grad = torch.empty(70, 50, device=dev)
+    error_d, x_d = error.to(dev), x.to(dev)
+    _lib.call('noise_reassemble', _lib.ptr(error_d), 70, _lib.ptr(x_d), 0, 50, 40, 70, 50, 1.0, _lib.ptr(grad),
+              _lib.stream(dev))
+    want = (error.double().t() @ x.double()).float()  # back to fp32: what overflows is infinite
+    got = grad.cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and got[20].isnan().all() and got[10, 6].isnan()
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    size = (error.abs().double().t() @ x.double())[fine]
+    assert fine[30, 4] and ((got[fine].double() - want[fine].double()).abs() <= 42 * 2.0 ** -24 * size).all()
+
+
 def test_adamw_matches_torch(dev):
     from noise_amd.optim import AdamW
     g = torch.Generator().manual_seed(2)
