@@ -11,10 +11,21 @@
 // centered over the batch when b > 1. The error of the slab's columns is -(sum over its draws of reward / sigma * a)
 // / (draws per slab); columns past the vocabulary are 0.
 //
-// Four launches, all of them element-parallel:
-//   head_prep_kernel    one wave per token row: capped logits, the 16 slab sums of exp, their total, the target logit
-//   head_loss_kernel    one wave per (draw, row): the 256 jittered columns (4 per lane, one Philox call), the CE
-//   head_center_kernel  one thread per (draw, position): rewards, centered over the batch
+// The reward of draw g at a row is c0 - log1p((e_g - e) / total) [+ z_g - z of a target inside the slab], with e_g the
+// slab's jittered exponential sum, e its clean one, and c0 = clean loss - log(total) + z formed once per row in float64:
+// a difference of the draws' small terms instead of one of two losses near 8, whose rounding was the larger part of the
+// estimate's error.
+//
+//   head_prep_kernel    one wave per token row: the slab sums of exp, their total, c0; zeros past the vocabulary
+//   head_error_kernel   one workgroup per (position, slab), a wave per batch row: every draw of the slab, from its jitter
+//                       (4 columns per lane, one Philox call) to the error sum. The jitter of 8 draws stays in registers
+//                       from the exponential sums to the weighted sum, the rewards' means over the batch go through LDS.
+//                       Bound by VALU issue (Philox and Box-Muller two thirds of it). 8 x 512 rows and 2,048 draws:
+//                       2.64 ms; 6.25 as a loss pass and an accumulation pass over stored [draws, rows] losses, each
+//                       making the jitter, with tanhf and expf per logit.
+// For batches of more rows than a workgroup has waves:
+//   head_reward_kernel  one wave per (draw, row): the reward
+//   head_center_kernel  one thread per (draw, position): the rewards centered over the batch
 //   head_accum_kernel   one wave per (row, slab): the draws of that slab regenerate their jitter, the error sum
 // The jitter is this library's counter stream (rng.h head_noise_quad), never stored.
 //
@@ -31,7 +42,26 @@ namespace noise {
 
 constexpr int kSlab = 256;
 
+constexpr int kHeadWaves = 16;  // waves of a head_error_kernel workgroup at most
+
 __device__ __forceinline__ float soft_cap(float x) { return 15.0f * tanhf(x / 15.0f); }
+
+// exp(15 tanh(x / 15) - 15) = exp2(g), g = -30 log2(e) / (exp(2 x / 15) + 1): three hardware exponentials and
+// reciprocals, about 3e-6 of the value. Only differences of sums of it enter the estimate.
+__device__ __forceinline__ float cap_exp(float x) {
+  constexpr float kIn = 2.0f / 15.0f * 1.4426950408889634f, kInv = 1.0f / (-30.0f * 1.4426950408889634f);
+  return fast_exp2(fast_rcp(fmaf(fast_exp2(x * kIn), kInv, kInv)));
+}
+
+// What the draws of a row share.
+struct HeadRow {
+  float slab_sum, inv_total, c0, z;
+  int tg;          // the target's column in the slab, -1 elsewhere
+  bool counted;    // not an ignored target
+  __device__ __forceinline__ float reward(float e, float zg) const {
+    return counted ? c0 - log1pf((e - slab_sum) * inv_total) + (tg >= 0 ? zg - z : 0.f) : 0.f;
+  }
+};
 
 // 4 bf16 (8 bytes) as floats
 __device__ __forceinline__ f32x4 ld_bf16x4(const bf16_t* p) {
@@ -40,106 +70,160 @@ __device__ __forceinline__ f32x4 ld_bf16x4(const bf16_t* p) {
 }
 
 __global__ __launch_bounds__(256) void head_prep_kernel(const bf16_t* __restrict__ raw, int64_t ld,
-                                                        const int64_t* __restrict__ targets, int64_t rows, int slabs,
+                                                        const int64_t* __restrict__ targets,
+                                                        const float* __restrict__ clean, int64_t rows, int slabs,
                                                         float* __restrict__ slab_sums, float* __restrict__ total,
-                                                        float* __restrict__ clean_t) {
+                                                        float* __restrict__ c0,
+                                                        float* __restrict__ error) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const bf16_t* r = raw + row * ld;
   const int64_t tg0 = targets[row];
   const int tg = tg0 < 0 ? 0 : (int)tg0;  // the reference clamps ignored targets to 0 (dust.py:275)
-  float tot = 0.f, tz = 0.f;
+  float tz = 0.f;
+  double tot = 0.0;
   for (int s = 0; s < slabs; ++s) {
-    const int c0 = s * kSlab + 4 * lane;
-    const f32x4 x = ld_bf16x4(r + c0);
+    const int at = s * kSlab + 4 * lane;
+    const f32x4 x = ld_bf16x4(r + at);
     float e = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float z = soft_cap(x[k]);
-      e += expf(z);
-      if (c0 + k == tg) tz = z;
+      e += cap_exp(x[k]);
+      if (at + k == tg) tz = soft_cap(x[k]);
     }
     const float se = warp_sum(e);
     if (lane == 0) slab_sums[row * slabs + s] = se;
-    tot += se;
+    tot += (double)se;
   }
   tz = warp_sum(tz);  // one lane holds the target logit, the others 0
   if (lane == 0) {
-    total[row] = tot;
-    clean_t[row] = tz;
+    total[row] = (float)tot;
+    c0[row] = (float)((double)clean[row] - (log(tot) + 15.0) + (double)tz);
   }
+  for (int64_t c = (int64_t)slabs * kSlab + lane; c < ld; c += 64) error[row * ld + c] = 0.f;  // past the vocabulary
 }
 
-__global__ __launch_bounds__(256) void head_loss_kernel(const bf16_t* __restrict__ raw, int64_t ld,
-                                                        const int64_t* __restrict__ targets, int64_t rows, int slabs,
-                                                        int n, float sigma, uint64_t seed,
-                                                        const float* __restrict__ slab_sums,
-                                                        const float* __restrict__ total,
-                                                        const float* __restrict__ clean_t, float* __restrict__ loss) {
+__device__ __forceinline__ HeadRow head_row(const bf16_t* raw, int64_t ld, const int64_t* targets,
+                                            const float* slab_sums, const float* total, const float* c0, int64_t row,
+                                            int slabs, int slab) {
+  const int64_t tg0 = targets[row], tg = (tg0 < 0 ? 0 : tg0) - (int64_t)slab * kSlab;
+  const bool in = tg >= 0 && tg < kSlab;
+  return HeadRow{slab_sums[row * slabs + slab], 1.0f / total[row], c0[row],
+                 in ? soft_cap(bf16_to_f32(raw[row * ld + slab * kSlab + tg])) : 0.f, in ? (int)tg : -1, tg0 != -1};
+}
+
+// error of the slab's 256 columns at the rows of position ti. Wave w: batch row w % b, and of the groups of 8 draws the
+// w / b-th of every `parts` (more than one where rows and slabs leave the GPU idle; their sums are added in order).
+__global__ __launch_bounds__(64 * kHeadWaves) void head_error_kernel(
+    const bf16_t* __restrict__ raw, int64_t ld, const int64_t* __restrict__ targets, int b, int t, int slabs, int n,
+    int per_slab, int parts, float sigma, uint64_t seed, const float* __restrict__ slab_sums,
+    const float* __restrict__ total, const float* __restrict__ c0,
+    float* __restrict__ error) {
+  __shared__ float rewards[2][kHeadWaves][8];
+  __shared__ f32x4 sums[kHeadWaves][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bi = wave % b, part = wave / b;
+  const int slab = blockIdx.y;
+  const int64_t row = (int64_t)bi * t + blockIdx.x;
+  const HeadRow hr = head_row(raw, ld, targets, slab_sums, total, c0, row, slabs, slab);
+  const int tg = __builtin_amdgcn_readfirstlane(hr.tg);
+  const f32x4 x = ld_bf16x4(raw + row * ld + slab * kSlab + 4 * lane);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int groups = (per_slab + 7) / 8, trips = (groups + parts - 1) / parts;
+  for (int it = 0; it < trips; ++it) {
+    const int q0 = 8 * (it * parts + part);
+    float a[8][4], e[8], zt = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const int q = q0 + d;  // draw q of the slab: draw q % n of its chunk q / n, which is chunk (q / n) slabs + slab
+      head_noise_quad(seed, (uint32_t)((q / n * slabs + slab) * n + q % n), (uint32_t)row, (uint32_t)lane, a[d]);
+      e[d] = 0.f;
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[k] = fmaf(sigma, a[d][k], x[k]);
+        e[d] += cap_exp(v[k]);
+      }
+      if (tg >= 0) {  // the jittered target, in the lanes of the draw's sum below
+        const float vt = lane_val(tg & 2 ? (tg & 1 ? v[3] : v[2]) : (tg & 1 ? v[1] : v[0]), tg >> 2);
+        zt = (lane >> 3) == d ? vt : zt;
+      }
+    }
+    const float es = warp_sum8(e, lane);  // lanes 8 d .. 8 d + 7: draw d
+    float rw = hr.reward(es, tg >= 0 ? soft_cap(zt) : 0.f);
+    if (b > 1) {
+      float (*buf)[8] = rewards[it & 1];  // the other buffer's readers are past the barrier of the trip between
+      if ((lane & 7) == 0) buf[wave][lane >> 3] = rw;
+      __syncthreads();
+      float mean = 0.f;
+      for (int k = 0; k < b; ++k) mean += buf[part * b + k][lane >> 3];
+      rw -= mean / (float)b;
+    }
+    const float w = q0 + (lane >> 3) < per_slab ? rw / sigma : 0.f;  // past the last draw: no weight
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const float wd = lane_val(w, 8 * d);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[k] = fmaf(wd, a[d][k], acc[k]);
+    }
+  }
+  if (parts > 1) {
+    sums[wave][lane] = acc;
+    __syncthreads();
+    if (part != 0) return;
+    for (int p = 1; p < parts; ++p) acc += sums[p * b + bi][lane];
+  }
+  const float inv = -1.0f / (float)per_slab;
+  *(f32x4*)(error + row * ld + slab * kSlab + 4 * lane) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+}
+
+__global__ __launch_bounds__(256) void head_reward_kernel(const bf16_t* __restrict__ raw, int64_t ld,
+                                                          const int64_t* __restrict__ targets, int64_t rows, int slabs,
+                                                          int n, float sigma, uint64_t seed,
+                                                          const float* __restrict__ slab_sums,
+                                                          const float* __restrict__ total,
+                                                          const float* __restrict__ c0, float* __restrict__ reward) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const uint32_t g = blockIdx.y;  // draw
   if (row >= rows) return;
-  const int block = (int)(g / (uint32_t)n) % slabs, lo = block * kSlab;
+  const int slab = (int)(g / (uint32_t)n) % slabs;
+  const HeadRow hr = head_row(raw, ld, targets, slab_sums, total, c0, row, slabs, slab);
   float a[4];
   head_noise_quad(seed, g, (uint32_t)row, (uint32_t)lane, a);
-  const f32x4 x = ld_bf16x4(raw + row * ld + lo + 4 * lane);
-  const int64_t tg0 = targets[row];
-  const int tg = tg0 < 0 ? 0 : (int)tg0;
-  float e = 0.f, tz = 0.f;
+  const f32x4 x = ld_bf16x4(raw + row * ld + slab * kSlab + 4 * lane);
+  float e = 0.f, zt = 0.f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float z = soft_cap(x[k] + sigma * a[k]);
-    e += expf(z);
-    if (lo + 4 * lane + k == tg) tz = z;
+    const float v = fmaf(sigma, a[k], x[k]);
+    e += cap_exp(v);
+    if (4 * lane + k == hr.tg) zt = soft_cap(v);
   }
-  e = warp_sum(e);
-  tz = warp_sum(tz);
-  if (lane == 0) {
-    const float part = (total[row] - slab_sums[row * slabs + block]) + e;
-    const bool in_slab = tg >= lo && tg < lo + kSlab;
-    loss[(int64_t)g * rows + row] = logf(part) - (in_slab ? tz : clean_t[row]);
-  }
+  const float rw = hr.reward(warp_sum(e), warp_sum(zt));
+  if (lane == 0) reward[(int64_t)g * rows + row] = rw;
 }
 
-// reward[g, r] = (target[r] != -1) ? clean[r] - loss[g, r] : 0, minus its mean over the batch (rows bi * t + ti)
-__global__ __launch_bounds__(256) void head_center_kernel(const int64_t* __restrict__ targets,
-                                                          const float* __restrict__ clean, int b, int t, int draws,
-                                                          float* __restrict__ loss) {
+// reward[g, r] minus its mean over the batch (rows bi * t + ti; b > 1)
+__global__ __launch_bounds__(256) void head_center_kernel(int b, int t, int draws, float* __restrict__ reward) {
   const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (id >= (int64_t)draws * t) return;
   const int64_t g = id / t, ti = id % t, rows = (int64_t)b * t;
-  float* lg = loss + g * rows;
+  float* rg = reward + g * rows + ti;
   float mean = 0.f;
-  for (int bi = 0; bi < b; ++bi) {
-    const int64_t r = (int64_t)bi * t + ti;
-    const float rw = targets[r] != -1 ? clean[r] - lg[r] : 0.f;
-    lg[r] = rw;
-    mean += rw;
-  }
-  if (b > 1) {
-    mean /= (float)b;
-    for (int bi = 0; bi < b; ++bi) lg[(int64_t)bi * t + ti] -= mean;
-  }
+  for (int bi = 0; bi < b; ++bi) mean += rg[(int64_t)bi * t];
+  mean /= (float)b;
+  for (int bi = 0; bi < b; ++bi) rg[(int64_t)bi * t] -= mean;
 }
 
 __global__ __launch_bounds__(256) void head_accum_kernel(const float* __restrict__ reward, int64_t rows, int64_t ld,
-                                                         int slabs, int n_slab_ld, int n, int chunks, float sigma,
-                                                         float inv_per_slab, uint64_t seed,
-                                                         float* __restrict__ error) {
+                                                         int slabs, int n, int chunks, float sigma, float inv_per_slab,
+                                                         uint64_t seed, float* __restrict__ error) {
   const int lane = threadIdx.x & 63;
   const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= rows * n_slab_ld) return;
-  const int64_t row = w / n_slab_ld;
-  const int slab = (int)(w % n_slab_ld), c0 = slab * kSlab + 4 * lane;
-  float* out = error + row * ld;
-  if (slab >= slabs) {  // past the vocabulary
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (c0 + k < ld) out[c0 + k] = 0.f;
-    return;
-  }
+  if (w >= rows * slabs) return;
+  const int64_t row = w / slabs;
+  const int slab = (int)(w % slabs);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   for (int c = slab; c < chunks; c += slabs)
     for (int j = 0; j < n; ++j) {
@@ -150,8 +234,8 @@ __global__ __launch_bounds__(256) void head_accum_kernel(const float* __restrict
 #pragma unroll
       for (int k = 0; k < 4; ++k) acc[k] += wgt * a[k];
     }
-  *(f32x4*)(out + c0) = f32x4{-acc[0] * inv_per_slab, -acc[1] * inv_per_slab, -acc[2] * inv_per_slab,
-                              -acc[3] * inv_per_slab};
+  *(f32x4*)(error + row * ld + slab * kSlab + 4 * lane) =
+      f32x4{-acc[0] * inv_per_slab, -acc[1] * inv_per_slab, -acc[2] * inv_per_slab, -acc[3] * inv_per_slab};
 }
 
 // reward[j, r] = clean[r] - loss[j, r], minus its mean over the chunk's n draws (n > 1) (dust.py:246-249)
@@ -248,26 +332,34 @@ extern "C" int noise_head_error(const uint16_t* raw, int64_t ld, const int64_t* 
   p += al256h((size_t)rows * slabs * 4);
   float* total = (float*)p;
   p += al256h((size_t)rows * 4);
-  float* clean_t = (float*)p;
+  float* c0 = (float*)p;
   p += al256h((size_t)rows * 4);
-  float* loss = (float*)p;
+  float* reward = (float*)p;
   const unsigned row_blocks = (unsigned)((rows + 3) / 4);
   const bf16_t* r = (const bf16_t*)raw;
   NoiseTimer tm(kTimeHeadError, stream);
-  hipLaunchKernelGGL(head_prep_kernel, dim3(row_blocks), dim3(256), 0, stream, r, ld, targets, rows, slabs, slab_sums,
-                     total, clean_t);
+  hipLaunchKernelGGL(head_prep_kernel, dim3(row_blocks), dim3(256), 0, stream, r, ld, targets, clean_loss, rows, slabs,
+                     slab_sums, total, c0, error);
   NOISE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(head_loss_kernel, dim3(row_blocks, (unsigned)draws), dim3(256), 0, stream, r, ld, targets, rows,
-                     slabs, n, sigma, seed, slab_sums, total, clean_t, loss);
+  if (b <= kHeadWaves) {
+    const int per_slab = draws / slabs;
+    // two waves per row and slab, or more, until the GPU's 1,024 SIMDs have about 4 each
+    int parts = 1;
+    while (2 * parts * b <= kHeadWaves && rows * slabs * parts < 4096 && 16 * parts < per_slab) parts *= 2;
+    hipLaunchKernelGGL(head_error_kernel, dim3((unsigned)t, (unsigned)slabs), dim3(64 * b * parts), 0, stream, r, ld,
+                       targets, b, t, slabs, n, per_slab, parts, sigma, seed, slab_sums, total, c0, error);
+    NOISE_LAUNCH_CHECK();
+    return NOISE_OK;
+  }
+  hipLaunchKernelGGL(head_reward_kernel, dim3(row_blocks, (unsigned)draws), dim3(256), 0, stream, r, ld, targets, rows,
+                     slabs, n, sigma, seed, slab_sums, total, c0, reward);
   NOISE_LAUNCH_CHECK();
   const int64_t nct = (int64_t)draws * t;
-  hipLaunchKernelGGL(head_center_kernel, dim3((unsigned)((nct + 255) / 256)), dim3(256), 0, stream, targets,
-                     clean_loss, b, t, draws, loss);
+  hipLaunchKernelGGL(head_center_kernel, dim3((unsigned)((nct + 255) / 256)), dim3(256), 0, stream, b, t, draws, reward);
   NOISE_LAUNCH_CHECK();
-  const int n_slab_ld = (int)((ld + kSlab - 1) / kSlab);
-  const int64_t waves = rows * n_slab_ld;
-  hipLaunchKernelGGL(head_accum_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, loss, rows, ld, slabs,
-                     n_slab_ld, n, chunks, sigma, 1.0f / (float)(draws / slabs), seed, error);
+  const int64_t waves = rows * slabs;
+  hipLaunchKernelGGL(head_accum_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, reward, rows, ld, slabs,
+                     n, chunks, sigma, 1.0f / (float)(draws / slabs), seed, error);
   NOISE_LAUNCH_CHECK();
   return NOISE_OK;
 }

@@ -39,6 +39,26 @@ def test_head_error_matches_oracle(dev, b, t, vocab, Vp, draws, nrep):
     assert torch.all(got[..., vocab:] == 0)
 
 
+@pytest.mark.parametrize('b,t,vocab,Vp,draws,nrep', [
+    (1, 8, 512, 512, 34, 17),    # a wave per row and slab with its draws in parts: 17 draws of a slab, in groups of 8
+    (3, 5, 256, 260, 7, 7),      # fewer draws than one group, 4 padded columns
+    (16, 4, 512, 768, 40, 4),    # as many batch rows as a workgroup has waves
+    (17, 4, 512, 512, 40, 4),    # one more: the rewards are stored
+])
+def test_head_error_batch_and_draw_edges(dev, b, t, vocab, Vp, draws, nrep):
+    """The waves of a (position, slab) workgroup: batch rows beside parts of the draws, groups of 8 draws that end early,
+    and the batches that do not fit one workgroup."""
+    print(f'head_error edges b={b} t={t} vocab={vocab} ld={Vp} draws={draws} nrep={nrep}', flush=True)
+    from noise_amd import dust
+    raw, y, clean = _case(b, t, Vp, seed=b * 1000 + t, vocab=vocab)
+    ref = od.head_error(raw, y, clean, draws, sigma=0.1, nrep=nrep, seed=9, vocab=vocab)
+    got = dust.head_error(raw.to(dev), y.to(dev), clean.to(dev), draws, sigma=0.1, nrep=nrep, seed=9,
+                          vocab=vocab).cpu()
+    err = ((got - ref).abs().max() / ref.abs().max()).item()
+    assert err < 1e-3, err
+    assert torch.all(got[..., vocab:] == 0)
+
+
 def test_head_error_rejects_uneven_slabs(dev):
     from noise_amd import dust
     raw, y, clean = _case(1, 16, 512, seed=1)
