@@ -855,6 +855,18 @@ using FcTile = GemmShape<256, 256, 64, 4, 2, 2, 1>;
 // Whole 512-wide rows, for the epilogues that normalize (both projections). attn_proj (K = 512) ran on 64 x 512 tiles
 // at two workgroups per CU with 32-deep steps before: 1.41 ms per C4 launch against 1.34 on this tile.
 using RowTile = GemmShape<128, 512, 64, 2, 4, 2>;
+// Few rows. The tiles above are then a handful of workgroups, each a serial chain of K steps with one or two steps of
+// loads in flight (128 rows: mlp_proj 64 us on one workgroup, attn_proj 23, c_fc 16 on 8, q|k|v 14 on 6), so smaller
+// tiles spread over more CUs and keep most of the LDS in flight: what a workgroup then costs is its operand bytes at
+// about 60 GB/s per CU (1.7 us of latency), a launch and its epilogue. Each serves while its workgroups are one round of
+// the 256 CUs; past that the next larger is faster (launch_tiles, launch_rows).
+using ShortTile32 = GemmShape<32, 256, 64, 1, 4, 4>;
+using ShortTile64 = GemmShape<64, 256, 64, 2, 4, 3>;
+using ShortTile128 = GemmShape<128, 256, 64, 2, 4, 3>;
+using StoreTile64 = GemmShape<64, 64, 64, 2, 2, 8>;
+using StoreTile64x128 = GemmShape<64, 128, 64, 2, 2, 6>;
+using StoreTile128 = GemmShape<128, 128, 64, 2, 2, 4>;
+constexpr int kCUs = 256;
 constexpr int kAttnOG = 1;  // 32 outputs per wave (4 waves per SIMD)
 
 static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -943,21 +955,70 @@ __global__ void member_rows_kernel(int32_t* __restrict__ seq, int64_t members, i
   if (m < members) seq[m] = (int32_t)(m % n_seq);
 }
 
+// C = A W^T to a staged epilogue, on the large tile S or, for few rows, on the short ones (us per launch, large / short:
+// q|k|v 14.4 / 8.7 at 128 rows, 15.9 / 10.5 at 2,048; c_fc 16.3 / 8.8, 18.6 / 10.2 and, 128-row tiles, 20 / 14.6 at
+// 4,096; the head 16.4 / 9.2, 19.5 / 17.2 at 2,048). q|k|v's epilogue is the heaviest and takes no 128-row short tile
+// (16.6 / 18.8 at 3,072).
+template <class S, class Epi>
+static hipError_t launch_tiles(const bf16_t* A, const bf16_t* W, int M, int N, int K, const Epi& epi, hipStream_t stream) {
+  constexpr bool kHeavy = std::is_same<Epi, EpiQKV>::value;
+  const int64_t tiles = (int64_t)(M + 127) / 128 * (N / 256);
+  if (4 * tiles <= kCUs) return launch_gemm<ShortTile32>(A, K, W, K, M, N, K, epi, stream);
+  if (2 * tiles <= kCUs) return launch_gemm<ShortTile64>(A, K, W, K, M, N, K, epi, stream);
+  if constexpr (!kHeavy)
+    if (tiles <= kCUs) return launch_gemm<ShortTile128>(A, K, W, K, M, N, K, epi, stream);
+  return launch_gemm<S>(A, K, W, K, M, N, K, epi, stream);
+}
+
+// C = A W^T [M, 512] to an epilogue of whole rows: inside the GEMM on 128 x 512 tiles, or, for few rows, stored in
+// `scratch` (bf16 [M, 512]) and read by the epilogue's own kernel (us, 128 x 512 / product + epilogue: mlp_proj 64 /
+// 9.9 + 5 at 128 rows, 64 / 17.5 + 7 at 4,096, 65 / 24.7 + 9.3 at 8,192; attn_proj 24 / 5.4 + 5, 24 / 9.3 + 7, 25 / 13.2
+// + 9.3; both together 100 / 106 at 16,384).
+template <class Epi>
+static hipError_t launch_rows(const bf16_t* A, const bf16_t* W, int M, int K, bf16_t* scratch, const Epi& epi,
+                              hipStream_t stream) {
+  const int panels = (M + 127) / 128;
+  const EpiStore st{scratch, kD, M};
+  hipError_t e;
+  if (16 * panels <= kCUs) e = launch_gemm<StoreTile64>(A, K, W, K, M, kD, K, st, stream);
+  else if (8 * panels <= kCUs) e = launch_gemm<StoreTile64x128>(A, K, W, K, M, kD, K, st, stream);
+  else if (4 * panels <= kCUs) e = launch_gemm<StoreTile128>(A, K, W, K, M, kD, K, st, stream);
+  else return launch_gemm<RowTile>(A, K, W, K, M, kD, K, epi, stream);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(epi_rows_kernel<Epi>, dim3((unsigned)((M + 4 * Epi::kRows - 1) / (4 * Epi::kRows))), dim3(256), 0,
+                     stream, scratch, M, epi);
+  return hipGetLastError();
+}
+
+// The large tile and the short ones of a staged epilogue.
+template <class S, class Epi>
+static hipError_t prepare_tiles() {
+  hipError_t e = prepare_gemm<S, Epi>();
+  if (e == hipSuccess) e = prepare_gemm<ShortTile32, Epi>();
+  if (e == hipSuccess) e = prepare_gemm<ShortTile64, Epi>();
+  if constexpr (!std::is_same<Epi, EpiQKV>::value)
+    if (e == hipSuccess) e = prepare_gemm<ShortTile128, Epi>();
+  return e;
+}
+
 static bool g_prepared = false;
 static int prepare_all() {
   if (g_prepared) return NOISE_OK;
-  NOISE_CHECK_HIP((prepare_gemm<Tile, EpiQKV>()));
+  NOISE_CHECK_HIP((prepare_tiles<Tile, EpiQKV>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<false, 1, false, false, true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<true, 3>>()));
-  NOISE_CHECK_HIP((prepare_gemm<FcTile, EpiReluSq>()));
-  NOISE_CHECK_HIP((prepare_gemm<FcTile, EpiReluSqT<true>>()));
+  NOISE_CHECK_HIP((prepare_tiles<FcTile, EpiReluSq>()));
+  NOISE_CHECK_HIP((prepare_tiles<FcTile, EpiReluSqT<true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<false, 1, true, false, true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<true, 3, true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<true, 3, false, true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<false, 1>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<false, 1, true>>()));
   NOISE_CHECK_HIP((prepare_gemm<RowTile, EpiResidNorm<false, 1, false, true, false, true>>()));
-  NOISE_CHECK_HIP((prepare_gemm<Tile, EpiHeadCE>()));
+  NOISE_CHECK_HIP((prepare_tiles<Tile, EpiHeadCE>()));
+  NOISE_CHECK_HIP((prepare_gemm<StoreTile64, EpiStore>()));
+  NOISE_CHECK_HIP((prepare_gemm<StoreTile64x128, EpiStore>()));
+  NOISE_CHECK_HIP((prepare_gemm<StoreTile128, EpiStore>()));
   g_prepared = true;
   return NOISE_OK;
 }
@@ -1104,7 +1165,7 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
               pert->ve[i], Vp, ws.rope};
     {
       NoiseTimer tm(kTimeQKV, stream);
-      NOISE_CHECK_HIP((launch_gemm<Tile>(ws.h, kD, L.w_qkv, kD, (int)M, kQKV, kD, eq, stream)));
+      NOISE_CHECK_HIP((launch_tiles<Tile>(ws.h, L.w_qkv, (int)M, kQKV, kD, eq, stream)));
     }
 
     FlashArgs fa;
@@ -1143,16 +1204,16 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
         EpiResidNorm<false, 1, true> ej;
         memcpy((void*)&ej, (const void*)&ep, sizeof(ep));
         ej.jit = jp;
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.y, kD, L.w_proj, kD, (int)M, kD, kD, ej, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.y, L.w_proj, (int)M, kD, ws.qkv, ej, stream)));
       } else if (i == 0 && x_from_x0) {
         EpiResidNorm<false, 1, false, true, false, true> eb;
         memcpy((void*)&eb, (const void*)&ep, sizeof(ep));
         eb.wte = model->wte; eb.x0_inv = ws.x0_inv; eb.Vp = Vp; eb.off_wte = pert->wte;
         eb.resid_lambdas = model->resid_lambdas; eb.x0_lambdas = model->x0_lambdas; eb.layer = 0;
         eb.off_resid = pert->resid_lambdas; eb.off_x0 = pert->x0_lambdas;
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.y, kD, L.w_proj, kD, (int)M, kD, kD, eb, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.y, L.w_proj, (int)M, kD, ws.qkv, eb, stream)));
       } else {
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.y, kD, L.w_proj, kD, (int)M, kD, kD, ep, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.y, L.w_proj, (int)M, kD, ws.qkv, ep, stream)));
       }
     }
 
@@ -1166,10 +1227,10 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
       const Jitter jf = dr->jit(i, 3);
       if (jf.on()) {
         EpiReluSqT<true> er{mb, ws.hid, kF, pert->c_fc[i], ws.xb, 4, pert->mlp_proj[i] + kD, ws.xb1, kF / Tile::BN, jf};
-        NOISE_CHECK_HIP((launch_gemm<FcTile>(ws.h, kD, L.w_fc, kD, (int)M, kF, kD, er, stream)));
+        NOISE_CHECK_HIP((launch_tiles<FcTile>(ws.h, L.w_fc, (int)M, kF, kD, er, stream)));
       } else {
         EpiReluSq er{mb, ws.hid, kF, pert->c_fc[i], ws.xb, 4, pert->mlp_proj[i] + kD, ws.xb1, kF / Tile::BN, Jitter{}};
-        NOISE_CHECK_HIP((launch_gemm<FcTile>(ws.h, kD, L.w_fc, kD, (int)M, kF, kD, er, stream)));
+        NOISE_CHECK_HIP((launch_tiles<FcTile>(ws.h, L.w_fc, (int)M, kF, kD, er, stream)));
       }
     }
 
@@ -1191,9 +1252,9 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
         EpiResidNorm<false, 1, true, false, true> ej;
         memcpy((void*)&ej, (const void*)&em, sizeof(em));
         ej.jit = jm;
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.hid, kF, L.w_mlp_proj, kF, (int)M, kD, kF, ej, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.hid, L.w_mlp_proj, (int)M, kF, ws.qkv, ej, stream)));
       } else {
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.hid, kF, L.w_mlp_proj, kF, (int)M, kD, kF, em, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.hid, L.w_mlp_proj, (int)M, kF, ws.qkv, em, stream)));
       }
     } else {
       EpiResidNorm<true, 3> em;
@@ -1209,14 +1270,14 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
         EpiResidNorm<true, 3, true> ej;
         memcpy((void*)&ej, (const void*)&em, sizeof(em));
         ej.jit = jm;
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.hid, kF, L.w_mlp_proj, kF, (int)M, kD, kF, ej, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.hid, L.w_mlp_proj, (int)M, kF, ws.qkv, ej, stream)));
       } else if (x0_recompute) {
         EpiResidNorm<true, 3, false, true> ex;
         memcpy((void*)&ex, (const void*)&em, sizeof(em));
         ex.wte = model->wte; ex.x0_inv = ws.x0_inv; ex.Vp = Vp; ex.off_wte = pert->wte;
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.hid, kF, L.w_mlp_proj, kF, (int)M, kD, kF, ex, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.hid, L.w_mlp_proj, (int)M, kF, ws.qkv, ex, stream)));
       } else {
-        NOISE_CHECK_HIP((launch_gemm<RowTile>(ws.hid, kF, L.w_mlp_proj, kF, (int)M, kD, kF, em, stream)));
+        NOISE_CHECK_HIP((launch_rows(ws.hid, L.w_mlp_proj, (int)M, kF, ws.qkv, em, stream)));
       }
     }
   }
@@ -1226,7 +1287,7 @@ static int forward_impl(const noise_gpt* model, const noise_perturbation* pert, 
   EpiHeadCE eh{mb, pert->lm_head, ws.xb, 4, model->vocab, n_part, ws.psum, ws.tgt, tg, logits};
   {
     NoiseTimer tm(kTimeHead, stream);
-    NOISE_CHECK_HIP((launch_gemm<Tile>(ws.h, kD, model->lm_head, kD, (int)M, Vp, kD, eh, stream)));
+    NOISE_CHECK_HIP((launch_tiles<Tile>(ws.h, model->lm_head, (int)M, Vp, kD, eh, stream)));
   }
   if (targets && (loss_sum || token_loss)) {
     NoiseTimer tm(kTimeCeFinal, stream);

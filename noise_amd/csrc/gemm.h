@@ -56,14 +56,17 @@ struct GemmShape {
   static constexpr int kEpiLds = BM * kEpiLd * 2;         // the whole tile in bf16
   static constexpr int kLdsBytes = kMainLds > kEpiLds ? kMainLds : kEpiLds;
   static constexpr int kWaveRows = BM / kWaves;           // epilogue rows per wave
-  static_assert((BK == 32 || BK == 64) && WTN == 128 && (WTM == 128 || WTM == 64) && (kWaves == 4 || kWaves == 8),
-                "main loop: 4 or 8 waves of 128x128 or 64x128, K steps of 32 or 64");
+  // Wave tiles of 32 or 64 rows and columns, for few rows: a plainer main loop that keeps kStages - 1 steps in flight
+  static constexpr bool kShort = WTN != 128;
+  static_assert(kShort ? BK == 64 && WTN <= 64 && WTM <= 64 && (kWaves == 4 || kWaves == 8)
+                       : (BK == 32 || BK == 64) && (WTM == 128 || WTM == 64) && (kWaves == 4 || kWaves == 8),
+                "main loop: 4 or 8 waves of 128x128 or 64x128, K steps of 32 or 64; 4 or 8 waves of up to 64x64, steps of 64");
   static_assert(kADma * kWaves * kLoadRows == BM && kBDma * kWaves * kLoadRows == BN,
                 "row groups of one load split evenly over waves");
-  static_assert((BM == 256 && BN == 256) || (BM == 128 && BN == 512) || (BM == 128 && BN == 256) ||
+  static_assert(kShort || (BM == 256 && BN == 256) || (BM == 128 && BN == 512) || (BM == 128 && BN == 256) ||
                     (BM == 64 && BN == 512),
                 "tiles: 256x256, 128x512, 128x256 or 64x512");
-  static_assert(kStages >= 2 && kStages <= 4, "stages");
+  static_assert(kStages >= 2 && kStages <= (kShort ? 8 : 4), "stages");
   static_assert((kStages - 1) * kDma < 64, "loads in flight: the vmcnt field");
   static_assert(kLdsBytes * kMinBlocks <= 160 * 1024, "LDS");
 };
@@ -259,6 +262,13 @@ struct AccEpilogue : std::false_type {};
 template <class E>
 struct AccEpilogue<E, std::void_t<decltype(E::kAccEpilogue)>> : std::bool_constant<E::kAccEpilogue> {};
 
+// An accumulator epilogue with `static constexpr bool kTransposed = true` takes the transposed product, as the staged
+// ones do (four consecutive columns of one row per register quad).
+template <class E, class = void>
+struct TransposedAcc : std::false_type {};
+template <class E>
+struct TransposedAcc<E, std::void_t<decltype(E::kTransposed)>> : std::bool_constant<E::kTransposed> {};
+
 // A staged epilogue may define ready(Wave&): the arithmetic on begin()'s per-row loads, run once the accumulators are
 // staged. An instruction that uses a loaded value makes the wave wait for the load; in begin() that wait would come
 // before the staging, here the staging has covered the load's latency.
@@ -268,11 +278,33 @@ template <class E>
 struct HasReady<E, std::void_t<decltype(std::declval<const E&>().ready(std::declval<typename E::Wave&>()))>>
     : std::true_type {};
 
+// What a wave of a staged epilogue loads ahead of the staging: its per-row data and its first group's.
+template <class S, class Epi>
+struct EpiAhead {
+  typename Epi::Wave w;
+  typename Epi::Pre p;
+  __device__ __forceinline__ void start(const Epi& epi, int M, int m0, int n0, int wave, int lane) {
+    const int row_base = m0 + wave * S::kWaveRows;
+    if (row_base >= M) return;
+    epi.begin(row_base, n0, lane, min(S::kWaveRows, M - row_base), w);  // per-row loads by lane: lanes < nrows
+    epi.load(row_base, n0, lane, w, p);
+  }
+};
+template <class S, class Epi>
+struct EpiAheadOf {
+  typedef EpiAhead<S, Epi> type;
+};
+struct EpiNothing {
+  typedef EpiNothing type;
+  template <class Epi>
+  __device__ __forceinline__ void start(const Epi&, int, int, int, int, int) {}
+};
+
 // Epilogue through LDS (every functor without an accumulator epilogue).
 template <class S, class Epi>
-__device__ __forceinline__ void staged_epilogue(const Epi& epi, f32x16 (&acc)[S::TM][S::TN], unsigned char* smem_raw,
-                                                int M, int m0, int n0, int n_tile, int wave, int wm, int wn,
-                                                int lane) {
+__device__ __forceinline__ void staged_epilogue(const Epi& epi, EpiAhead<S, Epi>& ahead, f32x16 (&acc)[S::TM][S::TN],
+                                                unsigned char* smem_raw, int M, int m0, int n0, int n_tile, int wave,
+                                                int wm, int wn, int lane) {
   // The accumulators (transposed: four consecutive columns of one row per register quad) are rounded to bf16 -- the
   // rounding of the reference's bf16 autocast matmul output, to which it then adds its fp32 rank-1 term -- and staged
   // as the whole tile, 8 bytes per write; the row pitch BN + 4 puts the 32 rows of one write on distinct pairs of the
@@ -287,17 +319,14 @@ __device__ __forceinline__ void staged_epilogue(const Epi& epi, f32x16 (&acc)[S:
   //   rows<R>(row0, n0, n_tile, lane, const Wave&, const Pre&, v)  the group's arithmetic and stores, with
   //   v = f32x4[R] (256-column tiles) or f32x4[R][2] (512-column tiles: columns 4l.. and 256 + 4l..).
   // The wave's per-row loads and its first group's loads are issued before the accumulators are staged, so their
-  // memory latency runs behind the staging.
+  // memory latency runs behind the staging (behind the main loop for the short tiles).
   bf16_t* st = (bf16_t*)smem_raw;
   constexpr int R = Epi::kRows, G = S::kWaveRows / Epi::kRows, H = S::BN / 256;
-  static_assert(G % 2 == 0, "groups are processed in pairs");
+  static_assert(G % 2 == 0 || G == 1, "groups are processed in pairs");
   const int row_base = m0 + wave * S::kWaveRows;
-  typename Epi::Wave w;
-  typename Epi::Pre p0, p1;
-  if (row_base < M) {
-    epi.begin(row_base, n0, lane, min(S::kWaveRows, M - row_base), w);  // per-row loads by lane: lanes < nrows
-    epi.load(row_base, n0, lane, w, p0);
-  }
+  if constexpr (!S::kShort) ahead.start(epi, M, m0, n0, wave, lane);
+  typename Epi::Wave& w = ahead.w;
+  typename Epi::Pre &p0 = ahead.p, p1;
 #pragma unroll
   for (int i = 0; i < S::TM; ++i)
 #pragma unroll
@@ -313,6 +342,10 @@ __device__ __forceinline__ void staged_epilogue(const Epi& epi, f32x16 (&acc)[S:
   if (row_base >= M) return;
   if constexpr (HasReady<Epi>::value) epi.ready(w);
   const bf16_t* st_wave = st + wave * S::kWaveRows * S::kEpiLd;
+  if constexpr (G == 1) {
+    epi_group<S::kEpiLd, H>(epi, st_wave, row_base, n0, n_tile, lane, w, p0);
+    return;
+  }
 #pragma unroll 1
   for (int g = 0; g < G; g += 2) {
     const int r0 = row_base + g * R;
@@ -411,83 +444,169 @@ __global__ __launch_bounds__(S::kThreads, S::kMinBlocks) void gemm_nt_kernel(con
   constexpr int kTileStride = 32 * S::kRowBytes;  // bytes between the 32-row MFMA tiles of a stage
 
   f32x16 acc[S::TM][S::TN];  // first written by step 0's first MFMAs, which take a zero accumulator
-  constexpr bool kTr = !AccEpilogue<Epi>::value;  // staged epilogues take the transposed tile
+  typename std::conditional<AccEpilogue<Epi>::value, EpiNothing, EpiAheadOf<S, Epi>>::type::type ahead;
+  constexpr bool kTr = !AccEpilogue<Epi>::value || TransposedAcc<Epi>::value;  // staged epilogues: the transposed tile
 
-  // Prologue: steps 0 .. NS - 1 in flight; stage 0 visible; its first k-substep's fragments read.
+  if constexpr (S::kShort) {
+    // Few tiles, one or two per CU with a wave or two per SIMD, so a step's own latencies count: kStages - 1 steps of 64
+    // are in flight, and a step's fragments are read together while the step before is multiplied. One barrier per step:
+    // past it every wave has the fragments of step kt, whose stage the loads of step kt + kStages then refill.
 #pragma unroll
-  for (int s = 0; s < NS; ++s) dma(s, s);
-  wait_vmcnt_imm<(NS - 1) * S::kDma>();
-  lds_barrier();
-  bf16x8 fa[2][S::TM], fb[2][S::TN];  // fragments of alternate k-substeps
+    for (int i = 0; i < S::TM; ++i)
 #pragma unroll
-  for (int i = 0; i < S::TM; ++i) fa[0][i] = frag(fa_off[0] + i * kTileStride);
+      for (int j = 0; j < S::TN; ++j) acc[i][j] = f32x16{};
 #pragma unroll
-  for (int j = 0; j < S::TN; ++j) fb[0][j] = frag(fb_off[0] + j * kTileStride);
+    for (int s = 0; s < NS; ++s) dma(s, s);
+    // The epilogue's first loads (chains of a few dependent ones) run beside the first steps'. They only add to the loads
+    // in flight, so the counted waits below wait for no less.
+    ahead.start(epi, M, m0, n0, wave, lane);
+    bf16x8 fa[2][S::kSub][S::TM], fb[2][S::kSub][S::TN];
+    auto read = [&](int kt, auto set) {
+      constexpr int c = decltype(set)::value;
+      const int pb = (kt % NS) * kStage;
+#pragma unroll
+      for (int kk = 0; kk < S::kSub; ++kk) {
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i) fa[c][kk][i] = frag(fa_off[kk] + pb + i * kTileStride);
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) fb[c][kk][j] = frag(fb_off[kk] + pb + j * kTileStride);
+      }
+    };
+    auto step = [&](int kt, auto set) {
+      constexpr int c = decltype(set)::value;
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      wait_vmcnt_imm<(NS - 2) * S::kDma>();  // stage kt + 1 has landed
+      lds_barrier();
+      dma(kt + NS, kt % NS);
+      read(kt + 1, std::integral_constant<int, c ^ 1>{});  // past the last step: zeros
+      __builtin_amdgcn_sched_barrier(0);  // the reads go out ahead of the MFMAs that cover them
+#pragma unroll
+      for (int kk = 0; kk < S::kSub; ++kk)
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+          for (int j = 0; j < S::TN; ++j) acc[i][j] = mma<kTr>(fa[c][kk][i], fb[c][kk][j], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    wait_vmcnt_imm<(NS - 1) * S::kDma>();
+    lds_barrier();
+    read(0, std::integral_constant<int, 0>{});
+    for (int kt = 0; kt < nk; kt += 2) {  // K is a multiple of two steps (launch_gemm)
+      step(kt, std::integral_constant<int, 0>{});
+      step(kt + 1, std::integral_constant<int, 1>{});
+    }
+  } else {
 
-  // Step kt on stage kt % NS: for each k-substep but the last, read the next k-substep and multiply this one; wait
-  // for this wave's reads and for stage kt + 1's loads, barrier (everyone is then past its reads of stage kt, and
-  // stage kt + 1 is visible); refill stage kt % NS with step kt + NS; read the next step's k-substep 0 and multiply
-  // the last k-substep.
-  // The reads and loads of each part are spread between its MFMAs (one per MFMA), so that neither the LDS nor the
-  // texture-address queue sees a burst.
-  // Step 0 is peeled: its first MFMAs take the inline constant 0 as the accumulator, so the accumulators need no
-  // zeroing moves.
-  auto step = [&](int kt, auto first) {
-    const int pb = (kt % NS) * kStage;
+    // Prologue: steps 0 .. NS - 1 in flight; stage 0 visible; its first k-substep's fragments read.
 #pragma unroll
-    for (int kk = 0; kk + 1 < S::kSub; ++kk) {
-      const int nx = (kk + 1) & 1, cu = kk & 1;
+    for (int s = 0; s < NS; ++s) dma(s, s);
+    wait_vmcnt_imm<(NS - 1) * S::kDma>();
+    lds_barrier();
+    bf16x8 fa[2][S::TM], fb[2][S::TN];  // fragments of alternate k-substeps
 #pragma unroll
-      for (int i = 0; i < S::TM; ++i) fa[nx][i] = frag(fa_off[kk + 1] + pb + i * kTileStride);
+    for (int i = 0; i < S::TM; ++i) fa[0][i] = frag(fa_off[0] + i * kTileStride);
 #pragma unroll
-      for (int j = 0; j < S::TN; ++j) fb[nx][j] = frag(fb_off[kk + 1] + pb + j * kTileStride);
+    for (int j = 0; j < S::TN; ++j) fb[0][j] = frag(fb_off[0] + j * kTileStride);
+
+    // Step kt on stage kt % NS: for each k-substep but the last, read the next k-substep and multiply this one; wait
+    // for this wave's reads and for stage kt + 1's loads, barrier (everyone is then past its reads of stage kt, and
+    // stage kt + 1 is visible); refill stage kt % NS with step kt + NS; read the next step's k-substep 0 and multiply
+    // the last k-substep.
+    // The reads and loads of each part are spread between its MFMAs (one per MFMA), so that neither the LDS nor the
+    // texture-address queue sees a burst.
+    // Step 0 is peeled: its first MFMAs take the inline constant 0 as the accumulator, so the accumulators need no
+    // zeroing moves.
+    auto step = [&](int kt, auto first) {
+      const int pb = (kt % NS) * kStage;
+#pragma unroll
+      for (int kk = 0; kk + 1 < S::kSub; ++kk) {
+        const int nx = (kk + 1) & 1, cu = kk & 1;
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i) fa[nx][i] = frag(fa_off[kk + 1] + pb + i * kTileStride);
+#pragma unroll
+        for (int j = 0; j < S::TN; ++j) fb[nx][j] = frag(fb_off[kk + 1] + pb + j * kTileStride);
+#pragma unroll
+        for (int i = 0; i < S::TM; ++i)
+#pragma unroll
+          for (int j = 0; j < S::TN; ++j)
+            acc[i][j] = mma<kTr>(fa[cu][i], fb[cu][j], decltype(first)::value && kk == 0 ? f32x16{} : acc[i][j]);
+        first_half_schedule<S>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      wait_vmcnt_imm<(NS - 2) * S::kDma>();  // stage kt + 1 has landed (the loads of kt + 2, kt + 3 may still fly)
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      dma(kt + NS, kt % NS);
+      const int nb = ((kt + 1) % NS) * kStage;
+      constexpr int kLast = (S::kSub - 1) & 1;  // the last k-substep's fragment set; the next step's first goes in 0
+#pragma unroll
+      for (int i = 0; i < S::TM; ++i) fa[0][i] = frag(fa_off[0] + nb + i * kTileStride);
+#pragma unroll
+      for (int j = 0; j < S::TN; ++j) fb[0][j] = frag(fb_off[0] + nb + j * kTileStride);
 #pragma unroll
       for (int i = 0; i < S::TM; ++i)
 #pragma unroll
         for (int j = 0; j < S::TN; ++j)
-          acc[i][j] = mma<kTr>(fa[cu][i], fb[cu][j], decltype(first)::value && kk == 0 ? f32x16{} : acc[i][j]);
-      first_half_schedule<S>();
+          acc[i][j] = mma<kTr>(fa[kLast][i], fb[kLast][j], acc[i][j]);
+      second_half_schedule<S>();
       __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-    wait_vmcnt_imm<(NS - 2) * S::kDma>();  // stage kt + 1 has landed (the loads of kt + 2, kt + 3 may still fly)
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    dma(kt + NS, kt % NS);
-    const int nb = ((kt + 1) % NS) * kStage;
-    constexpr int kLast = (S::kSub - 1) & 1;  // the last k-substep's fragment set; the next step's first goes in 0
-#pragma unroll
-    for (int i = 0; i < S::TM; ++i) fa[0][i] = frag(fa_off[0] + nb + i * kTileStride);
-#pragma unroll
-    for (int j = 0; j < S::TN; ++j) fb[0][j] = frag(fb_off[0] + nb + j * kTileStride);
-#pragma unroll
-    for (int i = 0; i < S::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < S::TN; ++j)
-        acc[i][j] = mma<kTr>(fa[kLast][i], fb[kLast][j], acc[i][j]);
-    second_half_schedule<S>();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  step(0, std::true_type{});
-  for (int kt = 1; kt < nk; ++kt) step(kt, std::false_type{});
+    };
+    step(0, std::true_type{});
+    for (int kt = 1; kt < nk; ++kt) step(kt, std::false_type{});
+  }
   wait_vmcnt_imm<0>();  // the loads issued past the last step have landed
   __syncthreads();      // every wave is done with the stages before the epilogue reuses the LDS
 
   if constexpr (AccEpilogue<Epi>::value)
     epi.template acc_epilogue<S>(acc, smem_raw, m0, n0, m_tile, n_tile, wave, wm, wn, lane);
   else
-    staged_epilogue<S>(epi, acc, smem_raw, M, m0, n0, n_tile, wave, wm, wn, lane);
+    staged_epilogue<S>(epi, ahead, acc, smem_raw, M, m0, n0, n_tile, wave, wm, wn, lane);
 }
 
-// Row / column of accumulator element (i, j, r) for this lane.
-__device__ __forceinline__ int acc_row(int row0, int i, int r, int lane) {
-  return row0 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+// c = A B^T rounded to bf16, stored as it is: the products of the split epilogues (epi_rows_kernel).
+struct EpiStore {
+  static constexpr bool kAccEpilogue = true, kTransposed = true;
+  bf16_t* c;  // [M, ldc]
+  int ldc, M;
+  template <class S>
+  __device__ __forceinline__ void acc_epilogue(f32x16 (&acc)[S::TM][S::TN], unsigned char*, int m0, int n0, int, int, int,
+                                               int wm, int wn, int lane) const {
+#pragma unroll
+    for (int i = 0; i < S::TM; ++i) {
+      const int row = m0 + wm * S::WTM + i * 32 + (lane & 31);
+      if (row >= M) continue;
+#pragma unroll
+      for (int j = 0; j < S::TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(u32x2*)(c + (int64_t)row * ldc + n0 + wn * S::WTN + j * 32 + q * 8 + (lane >> 5) * 4) =
+              u32x2{pack_bf16x2(acc[i][j][4 * q], acc[i][j][4 * q + 1]),
+                    pack_bf16x2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
+    }
+  }
+};
+
+// A staged epilogue of 512-wide rows on rows that EpiStore wrote: one wave per group of Epi::kRows rows. The same
+// arithmetic on the same rounded values as in the GEMM, so the outputs are the same bits.
+template <class Epi>
+__global__ __launch_bounds__(256) void epi_rows_kernel(const bf16_t* __restrict__ c, int M, Epi epi) {
+  constexpr int R = Epi::kRows;
+  const int lane = threadIdx.x & 63;
+  const int row0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * R;
+  if (row0 >= M) return;
+  typename Epi::Wave w;
+  typename Epi::Pre p;
+  epi.begin(row0, 0, lane, R, w);
+  epi.load(row0, 0, lane, w, p);
+  if constexpr (HasReady<Epi>::value) epi.ready(w);
+  epi_group<512, 2>(epi, c + (int64_t)row0 * 512, row0, 0, 0, lane, w, p);
 }
-__device__ __forceinline__ int acc_col(int col0, int j, int lane) { return col0 + j * 32 + (lane & 31); }
 
 template <class S, class Epi>
 static inline hipError_t launch_gemm(const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, int M, int N, int K,
                                      const Epi& epi, hipStream_t stream) {
+  if (S::kShort && K % (2 * S::BK)) return hipErrorInvalidValue;
   dim3 grid((N + S::BN - 1) / S::BN, (M + S::BM - 1) / S::BM);
   hipLaunchKernelGGL((gemm_nt_kernel<S, Epi>), grid, dim3(S::kThreads), S::kLdsBytes, stream, A, lda, B, ldb, M, N,
                      K, epi);

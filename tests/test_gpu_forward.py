@@ -142,6 +142,38 @@ def test_population_embedding_noise_reaches_every_mix(dev):
     assert (d_got - d_ref).abs().max().item() < 0.01, (d_got, d_ref)
 
 
+@pytest.mark.parametrize('members', [1, 5, 11, 16, 17, 22, 33, 43, 64, 65])
+def test_few_members_give_the_bits_of_many(dev, members):
+    """The tiles chosen by row count (128 rows per member here; each count is at or just past a rule's edge: 4, 2 or 1
+    workgroups per 256-column tile of q|k|v, c_fc and the head, the products stored ahead of the row epilogues up to 8,192
+    rows) sum the same products in the same order: per-token losses and logits equal those of the same members among 96."""
+    from noise_amd.model import GPTConfig
+    from noise_amd.population import NoiseLayout, run_forward
+    ocfg, _ = _cfgs()
+    model = _model(dev, _weights(ocfg), GPTConfig(sequence_len=SEQ))
+    layout = NoiseLayout(model)
+    g = torch.Generator(device=dev).manual_seed(8)
+    rows = torch.randn(96, layout.stride, device=dev, generator=g)
+    idx = torch.randint(0, 4096, (3, 128), device=dev, generator=g)
+    seq = torch.arange(96, device=dev, dtype=torch.int32) % 3
+    row = torch.arange(96, device=dev, dtype=torch.int32)
+    sign = torch.where(row % 2 == 0, 0.01, -0.01).float()
+
+    def run(n):
+        return run_forward(model, idx, idx.roll(1, 1).contiguous(), seq[:n].contiguous(), noise=rows,
+                           member_row=row[:n].contiguous(), member_sign=sign[:n].contiguous(), layout=layout,
+                           want_logits=n <= 5, want_tokens=True)
+
+    print(f'few members: {members} x 128', flush=True)
+    few, many = run(members), run(96)
+    assert torch.equal(few['token_loss'], many['token_loss'][:members * 128])
+    assert torch.equal(few['loss_sum'], many['loss_sum'][:members])
+    if members <= 5:
+        ce = torch.nn.functional.cross_entropy(few['logits'], idx.roll(1, 1)[seq[:members].long()].reshape(-1),
+                                               reduction='none')
+        assert torch.allclose(ce, few['token_loss'], rtol=1e-5, atol=1e-5)
+
+
 def test_lowrank_matches_bruteforce(dev):
     """x (W + s a b^T)^T with the perturbed weight materialized, on the CPU."""
     from noise_amd.population import lowrank
