@@ -43,6 +43,9 @@ __global__ void offsets_kernel(uint64_t seed, uint64_t step, RowsArgs args, int6
   out[i] = offset_value(seed, step, (uint32_t)p, (uint32_t)d, range);
 }
 
+// Four floats at any float address: one 16-byte store (offsets are arbitrary, so a quad rarely starts 16-byte aligned).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // grid.y walks the directions; x walks the quad slots of every parameter of the row, densely. A thread finds its
 // parameter by a binary search over the slot table, which the workgroup first copies into LDS.
 __global__ __launch_bounds__(256) void rows_kernel(uint64_t seed, const int64_t* __restrict__ offsets, int64_t pairs,
@@ -73,10 +76,14 @@ __global__ __launch_bounds__(256) void rows_kernel(uint64_t seed, const int64_t*
     if (blk > ((off + (uint64_t)width - 1) >> 2)) continue;
     float z[4];
     buffer_quad(seed, blk, z);
+    const int64_t e = (int64_t)(4 * blk) - (int64_t)off;  // the quad's first value in the slice (negative in the first quad)
+    if (e >= 0 && e + 4 <= width) {
+      *(f32x4_any*)(dst + e) = f32x4_any{z[0], z[1], z[2], z[3]};
+      asm volatile("" ::: "memory");  // keeps the store whole: the branches would be merged into four
+    } else {
 #pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      const uint64_t i = 4 * blk + l;
-      if (i >= off && i < off + (uint64_t)width) dst[i - off] = z[l];
+      for (int l = 0; l < 4; ++l)
+        if (e + l >= 0 && e + l < width) dst[e + l] = z[l];
     }
   }
 }
