@@ -212,9 +212,6 @@ class Dust:
         if T % 128:
             raise ValueError(f'sequence length {T} must be a multiple of 128')
         s, keep, dev = model.packed()
-        cos, sin = model.rope_tables(T)
-        s.rope_cos, s.rope_sin = cos.data_ptr(), sin.data_ptr()
-        self._rope = (cos, sin)
         self.x, self.y = x.long().contiguous(), y.long().contiguous()
         self.batch, self.length = b, T
         L, D = model.config.n_layer, model.config.n_embd
@@ -287,8 +284,6 @@ class Dust:
                 raise ValueError(f'site {name!r} is not in block {entry}')
             mask |= 1 << sid
         s, keep, dev = model.packed()
-        cos, sin = self._rope
-        s.rope_cos, s.rope_sin = cos.data_ptr(), sin.data_ptr()
         b, T = self.batch, self.length
         d = _lib.NoiseDustDraws()
         d.entry = -1 if entry is None else int(entry)

@@ -14,6 +14,7 @@ from dataclasses import dataclass
 import torch
 from torch import nn
 from torch.nn import functional as F
+from torch.nn.modules import module as _module
 
 from . import _lib
 
@@ -57,7 +58,15 @@ def attention(q, k, v, window):
         raise ValueError(f'q {tuple(q.shape)}, k {tuple(k.shape)} and v {tuple(v.shape)} must match')
     dtype = q.dtype
     Tp = (T + 127) // 128 * 128
-    q, k, v = (F.pad(t.to(torch.bfloat16), (0, 0, 0, 0, 0, Tp - T)).contiguous() for t in (q, k, v))
+    if Tp == T:
+        q, k, v = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
+    else:
+        padded = torch.empty(3, B, Tp, H, D, dtype=torch.bfloat16, device=q.device)
+        with torch.no_grad():
+            padded[2, :, T:] = 0  # the padding's weights are 0, so its values must be finite; its scores are masked
+            for i, t in enumerate((q, k, v)):
+                padded[i, :, :T] = t
+        q, k, v = padded[0], padded[1], padded[2]
     out = torch.empty_like(q)
     _lib.call('noise_attention', _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, H, Tp, Tp * H * D, H * D, int(window),
               _lib.ptr(out), Tp * H * D, H * D, None, _lib.stream(q.device))
@@ -147,12 +156,21 @@ class Block(nn.Module):
         return x + self.mlp(norm(x))
 
 
-def _hooked(model):
-    """True when a forward hook or pre-hook sits on any submodule (or globally): the fused forward would skip it."""
-    from torch.nn.modules import module as _m
-    if _m._global_forward_hooks or _m._global_forward_pre_hooks:
-        return True
-    return any(m._forward_hooks or m._forward_pre_hooks for m in model.modules() if m is not model)
+def _scan(model):
+    """One walk over the modules: (whether a forward hook or pre-hook sits on any submodule, or globally, so that the
+    fused forward would skip it; the parameters' and rotary tables' addresses and versions, the key of the packed
+    operands)."""
+    hooked = bool(_module._global_forward_hooks or _module._global_forward_pre_hooks)
+    key, todo = [], [model]
+    while todo:
+        m = todo.pop()
+        hooked = hooked or (m is not model and bool(m._forward_hooks or m._forward_pre_hooks))
+        for p in m._parameters.values():
+            if p is not None:
+                key.append((p.data_ptr(), p._version))
+        todo.extend(c for c in m._modules.values() if c is not None)
+    key += [(b.data_ptr(), b._version) for b in (model.cos, model.sin)]
+    return hooked, tuple(key)
 
 
 class GPT(nn.Module):
@@ -234,10 +252,10 @@ class GPT(nn.Module):
         if self.lm_head.weight.shape[0] % 256 or self.lm_head.weight.shape[0] > 4096:
             raise ValueError('padded vocabulary must be a multiple of 256 and at most 4096')
 
-    def packed(self):
-        """bf16 GEMM operands, fp32 tables and the ctypes model struct; rebuilt when any parameter changed."""
-        params = list(self.parameters())
-        key = tuple((p.data_ptr(), p._version) for p in params)
+    def packed(self, key=None):
+        """bf16 GEMM operands, fp32 tables and the ctypes model struct; rebuilt when any parameter or rotary table
+        changed (key: _scan's, when the caller has it)."""
+        key = _scan(self)[1] if key is None else key
         if self._packed is not None and self._packed[0] == key:
             return self._packed[1]
         self.check_shape()
@@ -256,6 +274,8 @@ class GPT(nn.Module):
         keep['lm_head'] = bf(self.lm_head.weight)
         s.resid_lambdas, s.x0_lambdas = keep['resid'].data_ptr(), keep['x0l'].data_ptr()
         s.wte, s.lm_head = keep['wte'].data_ptr(), keep['lm_head'].data_ptr()
+        keep['cos'], keep['sin'] = self.rope_tables(self.rotary_seq_len)  # every length's tables are their first rows
+        s.rope_cos, s.rope_sin = keep['cos'].data_ptr(), keep['sin'].data_ptr()
         for i, block in enumerate(self.transformer.h):
             a, m = block.attn, block.mlp
             L = s.layers[i]
@@ -286,7 +306,8 @@ class GPT(nn.Module):
         a caller has registered hooks on submodules (Dust's capture does, train/val/dust.py:166-168), the forward
         runs module by module instead, under bf16 autocast, so every hook sees its module's input and output."""
         _lib.require_device(idx)
-        if _hooked(self):
+        hooked, key = _scan(self)
+        if hooked:
             return self._forward_modules(idx, targets, loss_reduction)
         B, T = idx.shape
         Tp = (T + 127) // 128 * 128
@@ -299,10 +320,11 @@ class GPT(nn.Module):
             if Tp != T:
                 tg = F.pad(tg, (0, Tp - T), value=-1)
             tg = tg.contiguous()
-        from .population import run_forward
-        out = run_forward(self, idx.contiguous(), tg, member_seq=torch.arange(B, device=idx.device, dtype=torch.int32),
-                          noise=None, want_logits=targets is None, want_tokens=loss_reduction == 'none',
-                          check_tables=False)
+        from .population import forward_packed
+        out = forward_packed(self, self.packed(key), idx.contiguous(), tg,
+                             torch.arange(B, device=idx.device, dtype=torch.int32), None, None, None, None,
+                             want_logits=targets is None, want_tokens=loss_reduction == 'none', want_sum=True,
+                             check_tables=False)
         if targets is None:
             return out['logits'].view(B, Tp, -1)[:, :T]
         if loss_reduction == 'none':

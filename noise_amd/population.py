@@ -38,6 +38,7 @@ class NoiseLayout:
         self.stride = col
         self.index = {n: i for i, n in enumerate(self.names)}
         self._widths_c = None
+        self._columns = {}  # n_layer -> the perturbation struct's columns, filled in by struct()
 
     @property
     def widths_c(self):
@@ -65,7 +66,14 @@ class NoiseLayout:
         return out
 
     def struct(self, rows, n_layer):
-        return perturbation_struct(rows, self.stride, self.cols(n_layer), n_layer)
+        """The noise_perturbation struct of these rows; the columns are laid out once per layout."""
+        columns = self._columns.get(n_layer)
+        if columns is None:
+            columns = self._columns[n_layer] = bytes(perturbation_struct(None, self.stride, self.cols(n_layer), n_layer))
+        s = _lib.NoisePerturbation.from_buffer_copy(columns)
+        if rows is not None:
+            s.rows, s.n_rows = rows.data_ptr(), rows.shape[0]
+        return s
 
 
 def perturbation_struct(rows, stride, cols, n_layer):
@@ -138,17 +146,22 @@ def run_forward(model, tokens, targets, member_seq, noise=None, member_row=None,
     noise: fp32 rows [n_rows, layout.stride] or None; member_row / member_sign: int32 / fp32 [members].
     check_tables: also check the table entries' ranges on the host (a sync); callers that build their own tables
     pass False (the kernels still turn an out-of-range member into a NaN loss)."""
-    s, keep, dev = model.packed()
+    return forward_packed(model, model.packed(), tokens, targets, member_seq, noise, member_row, member_sign, layout,
+                          want_logits, want_tokens, want_sum, check_tables)
+
+
+def forward_packed(model, packed, tokens, targets, member_seq, noise, member_row, member_sign, layout, want_logits,
+                   want_tokens, want_sum, check_tables):
+    """run_forward on the model's packed operands."""
+    s, keep, dev = packed
     n_seq, T = tokens.shape
     members = member_seq.numel()
-    cos, sin = model.rope_tables(T)
-    s.rope_cos, s.rope_sin = cos.data_ptr(), sin.data_ptr()
-    layout = layout or NoiseLayout(model)
-    if noise is None:
-        member_row = torch.zeros(members, dtype=torch.int32, device=dev)
-        member_sign = torch.zeros(members, dtype=torch.float32, device=dev)
+    if noise is not None:
+        layout = layout or NoiseLayout(model)
+    else:  # no perturbation: the kernels read neither table, so any pointer serves
+        member_row = member_sign = member_seq
     _check_tables(tokens, targets, member_seq, noise, member_row, member_sign, layout, dev, check_tables)
-    pert = layout.struct(noise, model.config.n_layer)
+    pert = _lib.NoisePerturbation() if noise is None else layout.struct(noise, model.config.n_layer)
     out = {}
     out['loss_sum'] = torch.empty(members, dtype=torch.float32, device=dev) if (targets is not None and want_sum) else None
     out['token_loss'] = torch.empty(members * T, dtype=torch.float32, device=dev) if want_tokens else None
