@@ -65,7 +65,7 @@ struct EpiLowrank {
         v[q][e] += k * w.a[e];
         ss[q] += v[q][e] * v[q][e];
       }
-      if (y) *(f32x4*)(y + (int64_t)(row0 + q) * ldy + n0 + 4 * lane) = v[q];
+      if (y) __builtin_nontemporal_store(v[q], (f32x4*)(y + (int64_t)(row0 + q) * ldy + n0 + 4 * lane));
     }
     if (part) {
       const float tot = warp_sum8(ss, lane);
@@ -74,19 +74,35 @@ struct EpiLowrank {
   }
 };
 
-// u[r] = bf16(x[r] . bf16(b_{r / T})), one wave per row.
+// u[r] = bf16(x[r] . bf16(b_{r / T})), kDotRows rows of one member per wave (T is a multiple of them), 8 channels per
+// lane and load: the rows' loads are in flight together and b is converted once. Bound by the read of x (24 x 640 rows of
+// 512: 9.6 us with one row per wave in 2-byte loads, 4.9 here).
+constexpr int kDotRows = 8;
 __global__ __launch_bounds__(256) void lowrank_dot_kernel(const bf16_t* __restrict__ x, int K, int T,
                                                           const float* __restrict__ noise, int64_t stride,
                                                           int64_t b_off, float* __restrict__ u, int64_t M) {
-  const int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= M) return;
+  const int64_t r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (int64_t)kDotRows;
+  if (r0 >= M) return;
   const int lane = threadIdx.x & 63;
-  const float* bv = noise + (r / T) * stride + b_off;
-  const bf16_t* xr = x + r * K;
-  float d = 0.f;
-  for (int c = lane; c < K; c += 64) d += bf16_to_f32(xr[c]) * bf16_to_f32(f32_to_bf16(bv[c]));
-  d = warp_sum(d);
-  if (lane == 0) u[r] = bf16_to_f32(f32_to_bf16(d));
+  const float* bv = noise + (r0 / T) * stride + b_off;
+  const bf16_t* xr = x + r0 * K;
+  float d[kDotRows];
+#pragma unroll
+  for (int q = 0; q < kDotRows; ++q) d[q] = 0.f;
+  for (int c = 8 * lane; c < K; c += 512) {
+    u32x4 p[kDotRows], bp;
+#pragma unroll
+    for (int q = 0; q < kDotRows; ++q) p[q] = *(const u32x4*)(xr + (int64_t)q * K + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bp[j] = pack_bf16x2(bv[c + 2 * j], bv[c + 2 * j + 1]);
+#pragma unroll
+    for (int q = 0; q < kDotRows; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[q] = dot2_bf16(p[q][j], bp[j], d[q]);
+  }
+  static_assert(kDotRows == 8, "warp_sum8 reduces 8 rows");
+  const float tot = warp_sum8(d, lane);
+  if ((lane & 7) == 0) u[r0 + (lane >> 3)] = bf16_to_f32(f32_to_bf16(tot));
 }
 
 // sumsq[m] = sum of the member's per-row partials: one workgroup per member, fixed order (deterministic).
@@ -178,6 +194,9 @@ __global__ __launch_bounds__(256) void shared_u_kernel(const bf16_t* __restrict_
 // per-element one 0.513 against 0.524), 32-deep steps in four otherwise.
 using LTile = GemmShape<256, 256, 32, 2, 2>;
 using LTile64 = GemmShape<256, 256, 64, 2, 2, 2>;
+// The staged epilogues (per-member x, the plain linear).
+using LinTile = GemmShape<128, 256, 32, 2, 2, 3, 2>;  // two workgroups per CU
+using WideTile = GemmShape<256, 256, 64, 4, 2, 2>;    // 8 waves of 64 x 128
 
 template <class Epi>
 static hipError_t launch_shared_gemm(const uint16_t* x, const uint16_t* w, int64_t T, int64_t in, int64_t out,
@@ -578,15 +597,25 @@ extern "C" int noise_lowrank(const uint16_t* x, int32_t x_shared, const uint16_t
   NOISE_REQUIRE(workspace && workspace_bytes >= noise_lowrank_workspace(m, T, in, out, 0), "workspace too small");
   float* u = (float*)workspace;
   float* part = (float*)((char*)workspace + al256((size_t)M * 4));
-  hipLaunchKernelGGL(lowrank_dot_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, stream, (const bf16_t*)x,
+  hipLaunchKernelGGL(lowrank_dot_kernel, dim3((unsigned)((M / kDotRows + 3) / 4)), dim3(256), 0, stream, (const bf16_t*)x,
                      (int)in, (int)T, noise, noise_stride, b_off, u, M);
   NOISE_LAUNCH_CHECK();
   EpiLowrank epi{(int)T, noise, noise_stride, a_off, sign, u, y, out, sumsq ? part : nullptr, (int)(out / LTile::BN)};
-  NOISE_CHECK_HIP((prepare_gemm<LTile, EpiLowrank>()));
   {
     NoiseTimer tm(kTimeLowrank, stream);
-    NOISE_CHECK_HIP((launch_gemm<LTile>((const bf16_t*)x, in, (const bf16_t*)w, in, (int)M, (int)out, (int)in, epi,
-                                        stream)));
+    // 128 x 256 tiles, two workgroups per CU, so one's stores run beside the other's products; past four rounds of
+    // 256 x 256 tiles those with 64-deep steps are faster (us, two per CU / 256 x 256 in 64-deep steps / in 32-deep: 24
+    // members x 640 rows, 512 -> 2048: 58.5 / 62.6 / 66.2, 2048 -> 512: 60.2 / 69.3 / 67.9; 48 x 512, 512 -> 4096: 172 /
+    // 167 / 173; 256 x 512, 512 -> 2048: 431 / 416 / 421)
+    auto launch = [&](auto tile) {
+      using S = decltype(tile);
+      const hipError_t e = prepare_gemm<S, EpiLowrank>();
+      if (e != hipSuccess) return e;
+      return launch_gemm<S>((const bf16_t*)x, in, (const bf16_t*)w, in, (int)M, (int)out, (int)in, epi, stream);
+    };
+    if (M / LTile::BM * (out / LTile::BN) <= 1024) NOISE_CHECK_HIP(launch(LinTile{}));
+    else if (in % WideTile::BK == 0) NOISE_CHECK_HIP(launch(WideTile{}));
+    else NOISE_CHECK_HIP(launch(LTile{}));
   }
   if (sumsq) {
     hipLaunchKernelGGL(member_part_sum_kernel, dim3((unsigned)m), dim3(256), 0, stream, part,
@@ -618,7 +647,6 @@ struct EpiLinear {
                                     (u32x2*)(y + (int64_t)(row0 + q) * ldy + n0 + 4 * lane));
   }
 };
-using LinTile = GemmShape<128, 256, 32, 2, 2, 3, 2>;  // two workgroups per CU
 }  // namespace noise
 
 extern "C" int noise_linear(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t M, int64_t in, int64_t out,

@@ -103,3 +103,31 @@ def test_shared_sumsq_config2(dev):
             print(f'{md} member {i}: S {s[i].item():.6e} oracle {want[j].item():.6e} member part {part:.4e} '
                   f'err {err:.3e}', flush=True)
             assert err < 1e-3 * part, (md, i, err, part)  # measured 2.4e-5 of the member part
+
+
+@pytest.mark.parametrize('m,T,n_in,n_out', [
+    (1, 128, 32, 256),     # the smallest: one tile, one K step
+    (3, 128, 544, 512),    # K not a multiple of 64 nor of a wave's 512 channels
+    (5, 384, 1056, 256),   # more than one pass over the channels
+    (131, 128, 64, 4096),  # past four rounds of 256 x 256 tiles: 64-deep steps; 128 rows past a 256-row tile
+    (131, 128, 96, 4096),  # the same with K not a multiple of 64
+])
+def test_per_member_lowrank_over_its_tiles(dev, m, T, n_in, n_out):
+    """The per-member perturbed linear on each of its tiles, against float64 of the same bf16 operands: the output is the
+    bf16-rounded product (2^-8 of it) plus a rank-1 term whose dot is rounded to bf16 too."""
+    print(f'lowrank m={m} T={T} {n_in}->{n_out}', flush=True)
+    from noise_amd.population import lowrank
+    g = torch.Generator(device=dev).manual_seed(m * T + n_in)
+    x = torch.randn(m, T, n_in, device=dev, generator=g).bfloat16()
+    w = torch.randn(n_out, n_in, device=dev, generator=g).bfloat16()
+    a, b = torch.randn(m, n_out, device=dev, generator=g), torch.randn(m, n_in, device=dev, generator=g)
+    sign = torch.where(torch.arange(m, device=dev) % 2 == 0, 0.5, -0.5).float()
+    y = lowrank(x, w, a, b, sign)
+    assert torch.isfinite(y).all()
+    for i in sorted({0, 1, m // 2, m - 2, m - 1} & set(range(m))):
+        xi, ai, bi = x[i].double(), a[i].bfloat16().double(), b[i].bfloat16().double()
+        c, u = xi @ w.double().t(), xi @ bi
+        want = c + float(sign[i]) * u[:, None] * ai
+        bound = 2.0 ** -8 * (c.abs() + 0.5 * u.abs()[:, None] * ai.abs()) \
+            + 2.0 ** -20 * (xi.abs() @ w.double().abs().t() + 0.5 * (xi.abs() @ bi.abs())[:, None] * ai.abs())
+        assert ((y[i].double() - want).abs() <= bound).all(), i
