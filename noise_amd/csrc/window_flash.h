@@ -116,13 +116,20 @@ constexpr int kFlashOccupancy = (MODE == kAttn && OPT) ? 4 : (MODE == kCredit &&
 
 // OPT: kAttn's and kLse's bounded softmax; kCredit's value source as bf16 high and low parts (otherwise the high part
 // only).
-template <int MODE, bool OPT, int OG>
-__global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flash_kernel(FlashArgs a) {
+// NG: groups of four waves that share the workgroup's outputs, group g taking the input tiles g, g + NG, ..., each with
+// its own LDS stages; their sums are merged at the end (flash_groups says when).
+template <int MODE, bool OPT, int OG, int NG>
+__global__ __launch_bounds__(256 * NG, (NG > 1 ? NG : kFlashOccupancy<MODE, OPT>)) void window_flash_kernel(FlashArgs a) {
   constexpr int kBO = FlashTile<OG>::BO;
-  __shared__ __align__(16) bf16_t ys[2][64 * 64];
-  __shared__ __align__(16) bf16_t vt_hi[2][64 * 64];
-  __shared__ __align__(16) bf16_t vt_lo[MODE == kCredit && OPT ? 2 : 1][MODE == kCredit && OPT ? 64 * 64 : 4];
-  __shared__ float lse_s[2][64];
+  __shared__ __align__(16) bf16_t ys_all[NG][2][64 * 64];
+  __shared__ __align__(16) bf16_t vt_hi_all[NG][2][64 * 64];
+  __shared__ __align__(16) bf16_t vt_lo_all[NG][MODE == kCredit && OPT ? 2 : 1][MODE == kCredit && OPT ? 64 * 64 : 4];
+  __shared__ float lse_s_all[NG][2][64];
+  const int group = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  auto& ys = ys_all[group];
+  auto& vt_hi = vt_hi_all[group];
+  auto& vt_lo = vt_lo_all[group];
+  auto& lse_s = lse_s_all[group];
 
   const int T = a.T, W = a.window;
   const int n_tiles = (T + kBO - 1) / kBO;
@@ -152,7 +159,7 @@ __global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flas
   const int head = (int)(row_idx % gridDim.y);
   const int64_t b = row_idx / gridDim.y;
   const int o0 = tile * kBO;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;  // within the group
   const int half = lane >> 5, col = lane & 31;
   const int ow = o0 + wave * 32 * OG;  // this wave's first output
   const bool wave_live = ow < T;       // T % 128 == 0, so a live wave's outputs are all < T
@@ -287,9 +294,12 @@ __global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flas
   };
 
   FlashStage<MODE> stage;
-  dma(i_begin, 0);
-  load(i_begin, stage);
-  store(0, stage);
+  const int i_first = i_begin + group * kFlashBI;  // this group's first tile (past i_end: it has none)
+  if (NG == 1 || i_first < i_end) {
+    dma(i_first, 0);
+    load(i_first, stage);
+    store(0, stage);
+  }
   __builtin_amdgcn_s_waitcnt(kWaitVm0);
   __syncthreads();
   // The x (and hub) fragments are loop-invariant registers whose loads may still be in flight here. Each iteration
@@ -311,23 +321,23 @@ __global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flas
     // after the first tile nothing counted by vmcnt is in flight here (each tile ends with vmcnt(0)); at the first,
     // this retires what the prologue left (spill stores), so that no wait inside the tile is for them
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    const bool more = i0 + kFlashBI < i_end;
+    const bool more = i0 + NG * kFlashBI < i_end;
     if (more) {
-      dma(i0 + kFlashBI, s ^ 1);
-      load(i0 + kFlashBI, stage);
+      dma(i0 + NG * kFlashBI, s ^ 1);
+      load(i0 + NG * kFlashBI, stage);
     }
 
     // per output group: any valid pair in this tile, and no pair masked
     bool any[OG], full[OG];
-    bool any_og = false;
+    bool any_og = false;  // a group's turn past its last tile has none
 #pragma unroll
     for (int og = 0; og < OG; ++og) {
       const int g0 = ow + og * 32;
       if (MODE == kCredit) {
-        any[og] = wave_live && (i0 + kFlashBI - 1 >= g0) && (i0 <= g0 + 31 + W);
+        any[og] = wave_live && (i0 + kFlashBI - 1 >= g0) && (i0 <= g0 + 31 + W) && (NG == 1 || i0 < i_end);
         full[og] = (i0 >= g0 + 31) && (i0 + kFlashBI - 1 <= g0 + W);
       } else {
-        any[og] = wave_live && (i0 <= g0 + 31) && (i0 + kFlashBI - 1 >= g0 - W);
+        any[og] = wave_live && (i0 <= g0 + 31) && (i0 + kFlashBI - 1 >= g0 - W) && (NG == 1 || i0 < i_end);
         full[og] = (i0 + kFlashBI - 1 <= g0) && (i0 >= g0 + 31 - W);
       }
       any_og = any_og || any[og];
@@ -543,12 +553,48 @@ __global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flas
     __builtin_amdgcn_s_waitcnt(kWaitVm0);  // the next tile has landed in LDS
     __syncthreads();
   };
-  for (int i0 = i_begin; i0 < i_end; i0 += 2 * kFlashBI) {
-    input_tile(i0, std::integral_constant<int, 0>{});
-    if (i0 + kFlashBI >= i_end) break;
-    input_tile(i0 + kFlashBI, std::integral_constant<int, 1>{});
+  for (int i0 = i_begin; i0 < i_end; i0 += 2 * NG * kFlashBI) {  // every group takes every turn (the barriers)
+    input_tile(i0 + group * kFlashBI, std::integral_constant<int, 0>{});
+    if (i0 + NG * kFlashBI >= i_end) break;
+    input_tile(i0 + (NG + group) * kFlashBI, std::integral_constant<int, 1>{});
   }
 
+  if constexpr (NG > 1) {
+    // Group 0 takes group 1's sums through the stages' LDS, free after the loop's last barrier.
+    static_assert(NG == 2 && OG == 1 && sizeof(ys_all) >= 4 * 32 * 64 * 4 && sizeof(vt_hi_all) >= 4 * 3 * 64 * 4,
+                  "four waves' accumulators fit ys, their row sums vt_hi");
+    float* acc_s = (float*)&ys_all[0][0][0] + wave * 32 * 64 + lane;
+    float* row_s = (float*)&vt_hi_all[0][0][0] + wave * 3 * 64 + lane;
+    constexpr bool has_acc = MODE == kAttn || MODE == kCredit;
+    if (group == 1) {
+      if constexpr (has_acc) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r) acc_s[r * 64] = o_acc[0][r >> 4][r & 15];
+      }
+      row_s[0] = m_run[0];
+      row_s[64] = l_run[0];
+      row_s[128] = c_run[0];
+    }
+    __syncthreads();
+    if (group == 0) {
+      float mine = 1.f, other = 1.f;  // the two groups' scales to their common maximum
+      if constexpr (!bounded && MODE != kCredit) {
+        const float m_new = fmaxf(m_run[0], row_s[0]), m_safe = m_new == -INFINITY ? 0.f : m_new;
+        mine = fast_exp2(m_run[0] - m_safe);
+        other = fast_exp2(row_s[0] - m_safe);
+        m_run[0] = m_new;
+      }
+      l_run[0] = l_run[0] * mine + row_s[64] * other;
+      c_run[0] = c_run[0] * mine + row_s[128] * other;
+      if constexpr (has_acc) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r)
+          o_acc[0][r >> 4][r & 15] = o_acc[0][r >> 4][r & 15] * mine + acc_s[r * 64] * other;
+      }
+    }
+    __syncthreads();  // group 0's attention output is staged in ys
+    if (group == 1) return;
+  }
   if (!wave_live) return;
   // ---- epilogue ----
 #pragma unroll
@@ -643,12 +689,37 @@ __global__ __launch_bounds__(256, (kFlashOccupancy<MODE, OPT>)) void window_flas
 
 namespace noise {
 
+// Groups of waves per workgroup. A wave's chain per input tile (LDS reads, MFMA latency, the exponentials) takes about
+// 0.7 us, with one wave per SIMD nothing covers it, and loads issued further ahead changed nothing; so where the longest
+// chain, not the work of all workgroups spread over the CUs, bounds the launch, two groups halve it. The line lies at a
+// mean load per CU of 7/8 of the longest chain, of at least 8 tiles (us with one / two groups; value pass with hi + lo
+// parts, attention; rows x T, window):
+//   mean / longest 0.17  3 x 2048, 2048: 36.5 / 29.1, 27.9 / 23.5     0.84  48 x 1024, 1024: 23.6 / 21.4, 18.0 / 17.2
+//                  0.53 16 x 2048, 2048: 37.3 / 30.2, 28.6 / 23.9     1.13  24 x 2048, 1024: 26.9 / 30.1, 22.7 / 23.3
+//                  0.75 32 x 1024,  512: 16.5 / 14.3, 13.3 / 11.8     1.59  48 x 2048, 2048: 52.8 / 60.7, 40.5 / 44.4
+// (4 tiles: 8 x 256: 13.4 / 13.3, 8.9 / 8.7). Four groups spill. The bounded attention of the forwards keeps one: a
+// member's loss has the same bits however many members run beside it.
+template <int OG>
+inline int flash_groups(int64_t T, int64_t window, int64_t rows) {
+  constexpr int64_t kBO = FlashTile<OG>::BO;
+  const int64_t longest = ((window < T ? window : T) + kBO + kFlashBI - 1) / kFlashBI;
+  int64_t total = 0;  // tiles of one row's workgroups
+  for (int64_t o = kBO; o < T + kBO; o += kBO) total += o / kFlashBI < longest ? o / kFlashBI : longest;
+  return longest >= 8 && T >= 8 * kFlashBI && total * rows * 8 <= longest * 256 * 7 ? 2 : 1;
+}
+
 // One launch of the flash kernel over `batch` x `heads` rows of T tokens (T % 128 == 0).
 template <int MODE, bool OPT, int OG>
 inline hipError_t launch_flash(const FlashArgs& a, int64_t batch, int heads, hipStream_t stream) {
   constexpr int kBO = FlashTile<OG>::BO;
-  hipLaunchKernelGGL((window_flash_kernel<MODE, OPT, OG>), dim3((unsigned)((a.T + kBO - 1) / kBO), (unsigned)heads,
-                     (unsigned)batch), dim3(256), 0, stream, a);
+  const dim3 grid((unsigned)((a.T + kBO - 1) / kBO), (unsigned)heads, (unsigned)batch);
+  if constexpr (MODE != kAttn || !OPT) {
+    if (flash_groups<OG>(a.T, a.window, batch * heads) == 2) {
+      hipLaunchKernelGGL((window_flash_kernel<MODE, OPT, OG, 2>), grid, dim3(512), 0, stream, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((window_flash_kernel<MODE, OPT, OG, 1>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -229,3 +229,35 @@ def test_attention_periodic_equals_replicated_operands(dev, bounded):
     ref = om.attention(qf[e:e + 1].float().cpu(), kf[e:e + 1].float().cpu(), v6[e:e + 1].float().cpu(), W)
     got = outs[0][e:e + 1].view(1, T, H, 64).float().cpu()
     assert _relmax(got, ref) < 2e-2
+
+
+@pytest.mark.parametrize('T,window', [(512, 320), (512, 321), (640, 512), (896, 449), (640, 640), (1536, 1024)])
+def test_two_groups_of_waves(dev, T, window):
+    """Few rows of long windows: two groups of waves share a workgroup's tiles (320 is the last window of one group),
+    with outputs of odd numbers of tiles, and of so few that the second group has none. Against float64 of the bf16
+    operands: a probability is rounded to bf16 (2^-9 of it, and as much again for the bf16 parts of a source or for the
+    bf16 output), the LSE is fp32."""
+    from noise_amd import credit
+    from noise_amd.model import attention
+    print(f'two groups T={T} window={window}', flush=True)
+    rows = 2
+    q, k = _qk(rows, T, True, seed=T + window)
+    v, hub = _bf(rows, T, 5), _bf(rows, T, 6)
+    src = torch.randn(rows, T, 64, generator=torch.Generator().manual_seed(7))
+    qd, kd, vd, hd, sd = (t.double() for t in (q, k, v, hub, src))
+    A, lse_ref = oc.attention_maps(qd, kd, window), oc.lse(qd, kd, window)
+    lse = credit.credit_lse(q.to(dev), k.to(dev), window)
+    assert (lse.cpu().double() - lse_ref).abs().max().item() < 1e-4
+    P = A.transpose(-1, -2)
+    for hi_lo in (False, True):
+        out = credit.raw_value_credits(q.to(dev), k.to(dev), lse, src.to(dev), window, hi_lo=hi_lo).cpu().double()
+        assert ((out - P @ sd).abs() <= 2.0 ** -7 * (P @ sd.abs()) + 1e-5).all(), hi_lo
+    lse2, center = (t.cpu().double() for t in credit.key_context(q.to(dev), k.to(dev), v.to(dev), hub.to(dev), window))
+    ref = (A * (hd @ vd.transpose(-1, -2))).sum(-1)
+    assert (lse2 - lse_ref).abs().max().item() < 1e-4
+    assert (center - ref).abs().max().item() < 1e-4 * ref.abs().max().item()
+    bounded = credit.credit_lse(q.to(dev), k.to(dev), window, True).cpu().double()
+    assert (bounded - lse_ref).abs().max().item() < 2e-2 + 2e-3 * 8
+    heads = lambda t: t.transpose(0, 1).unsqueeze(0).contiguous().to(dev)
+    out = attention(heads(q), heads(k), heads(v), window)[0].transpose(0, 1).cpu().double()
+    assert ((out - A @ vd).abs() <= 2.0 ** -7 * (A @ vd.abs()) + 1e-5).all()
