@@ -119,6 +119,10 @@ int noise_lowrank_static(const uint16_t* x, int32_t x_shared, const uint16_t* w,
 int noise_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t batch, int32_t heads, int64_t T,
                     int64_t stride_b, int64_t stride_t, int32_t window, uint16_t* out, int64_t out_stride_b,
                     int64_t out_stride_t, float* lse, void* stream);
+/* noise_attention for any T > 0: nothing has to be padded (and copied) to a multiple of 128. */
+int noise_attention_any_length(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t batch, int32_t heads,
+                               int64_t T, int64_t stride_b, int64_t stride_t, int32_t window, uint16_t* out,
+                               int64_t out_stride_b, int64_t out_stride_t, float* lse, void* stream);
 /* noise_attention with operands shared by groups of batch entries: with a period p > 0, batch entry e reads entry
  * e % p of that operand (0: its own), so draws stacked draw-major over a batch of p rows read one clean copy of the
  * operands they do not jitter. bounded != 0 uses the softmax without a running maximum, weights exp(s) with s = q . k / 8,

@@ -55,6 +55,8 @@ _SIGNATURES = {
     'noise_linear': ([c_p, i64, c_p, i64, i64, i64, c_p, i64, c_p], ctypes.c_int),
     'noise_lowrank_static': ([c_p, i32, c_p, c_p, i64, i64, i64, c_p, i64, i64, i64, i64, c_p, c_p, c_p], ctypes.c_int),
     'noise_attention': ([c_p, c_p, c_p, i64, i32, i64, i64, i64, i32, c_p, i64, i64, c_p, c_p], ctypes.c_int),
+    'noise_attention_any_length': ([c_p, c_p, c_p, i64, i32, i64, i64, i64, i32, c_p, i64, i64, c_p, c_p],
+                                   ctypes.c_int),
     'noise_population_forward_workspace': ([i64, i64], szt),
     'noise_population_forward': ([ctypes.POINTER(NoiseGpt), ctypes.POINTER(NoisePerturbation), c_p, c_p, i64, i64,
                                   c_p, c_p, c_p, i64, c_p, c_p, c_p, c_p, szt, c_p], ctypes.c_int),

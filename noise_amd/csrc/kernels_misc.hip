@@ -5,12 +5,13 @@
 
 using namespace noise;
 
-extern "C" int noise_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t batch, int32_t heads,
-                               int64_t T, int64_t stride_b, int64_t stride_t, int32_t window, uint16_t* out,
-                               int64_t out_stride_b, int64_t out_stride_t, float* lse, void* stream) {
+extern "C" int noise_attention_any_length(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t batch,
+                                          int32_t heads, int64_t T, int64_t stride_b, int64_t stride_t, int32_t window,
+                                          uint16_t* out, int64_t out_stride_b, int64_t out_stride_t, float* lse,
+                                          void* stream) {
   NOISE_REQUIRE(q && k && v && out, "NULL pointer argument");
   NOISE_REQUIRE(batch > 0 && batch <= 65535 && heads > 0 && heads <= 65535, "batch / heads outside [1, 65535]");
-  NOISE_REQUIRE(T > 0 && T % 128 == 0, "T = %lld must be a positive multiple of 128", (long long)T);
+  NOISE_REQUIRE(T > 0 && T <= INT32_MAX - 256, "T = %lld must be positive", (long long)T);
   NOISE_REQUIRE(window >= 0, "negative window");
   NOISE_REQUIRE(stride_t % 8 == 0 && stride_b % 8 == 0 && out_stride_t % 4 == 0, "strides must keep 16-byte rows");
   FlashArgs a;
@@ -24,6 +25,14 @@ extern "C" int noise_attention(const uint16_t* q, const uint16_t* k, const uint1
   NoiseTimer tm(kTimeAttention, (hipStream_t)stream);
   NOISE_CHECK_HIP((launch_flash<kAttn, false, 1>(a, batch, heads, (hipStream_t)stream)));
   return NOISE_OK;
+}
+
+extern "C" int noise_attention(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t batch, int32_t heads,
+                               int64_t T, int64_t stride_b, int64_t stride_t, int32_t window, uint16_t* out,
+                               int64_t out_stride_b, int64_t out_stride_t, float* lse, void* stream) {
+  NOISE_REQUIRE(T > 0 && T % 128 == 0, "T = %lld must be a positive multiple of 128", (long long)T);
+  return noise_attention_any_length(q, k, v, batch, heads, T, stride_b, stride_t, window, out, out_stride_b,
+                                    out_stride_t, lse, stream);
 }
 
 extern "C" int noise_attention_periodic(const uint16_t* q, int32_t q_period, const uint16_t* k, int32_t k_period,

@@ -48,8 +48,7 @@ def apply_rotary_emb(x, cos, sin):
 
 def attention(q, k, v, window):
     """Causal attention with a left window on [batch, token, head, 64] tensors (utils/model.py:24-31): the HIP
-    windowed flash kernel, bf16 operands, fp32 softmax statistics; the output in q's dtype. A length that is not a
-    multiple of 128 is padded at the end (causal: the padding never reaches a real position)."""
+    windowed flash kernel, bf16 operands, fp32 softmax statistics; the output in q's dtype."""
     _lib.require_device(q, k, v)
     B, T, H, D = q.shape
     if D != 64:
@@ -57,20 +56,12 @@ def attention(q, k, v, window):
     if k.shape != q.shape or v.shape != q.shape:
         raise ValueError(f'q {tuple(q.shape)}, k {tuple(k.shape)} and v {tuple(v.shape)} must match')
     dtype = q.dtype
-    Tp = (T + 127) // 128 * 128
-    if Tp == T:
-        q, k, v = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
-    else:
-        padded = torch.empty(3, B, Tp, H, D, dtype=torch.bfloat16, device=q.device)
-        with torch.no_grad():
-            padded[2, :, T:] = 0  # the padding's weights are 0, so its values must be finite; its scores are masked
-            for i, t in enumerate((q, k, v)):
-                padded[i, :, :T] = t
-        q, k, v = padded[0], padded[1], padded[2]
+    q, k, v = (t.to(torch.bfloat16).contiguous() for t in (q, k, v))
+    q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))  # the kernel reads 16 bytes at a time
     out = torch.empty_like(q)
-    _lib.call('noise_attention', _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, H, Tp, Tp * H * D, H * D, int(window),
-              _lib.ptr(out), Tp * H * D, H * D, None, _lib.stream(q.device))
-    return out[:, :T].to(dtype)
+    _lib.call('noise_attention_any_length', _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, H, T, T * H * D, H * D,
+              int(window), _lib.ptr(out), T * H * D, H * D, None, _lib.stream(q.device))
+    return out.to(dtype)
 
 
 def linear_bf16(x, weight):

@@ -261,3 +261,20 @@ def test_two_groups_of_waves(dev, T, window):
     heads = lambda t: t.transpose(0, 1).unsqueeze(0).contiguous().to(dev)
     out = attention(heads(q), heads(k), heads(v), window)[0].transpose(0, 1).cpu().double()
     assert ((out - A @ vd).abs() <= 2.0 ** -7 * (A @ vd.abs()) + 1e-5).all()
+
+
+@pytest.mark.parametrize('T,window', [(1, 0), (31, 31), (64, 5), (65, 64), (129, 200), (200, 100), (577, 577), (1001, 700)])
+def test_attention_any_length(dev, T, window):
+    """Lengths that end inside a tile of 64 inputs, of 128 outputs or of a wave's 32, one and two groups of waves, and an
+    operand that starts off a 16-byte boundary. Bound: the probabilities and the output rounded to bf16."""
+    from noise_amd.model import attention
+    print(f'attention T={T} window={window}', flush=True)
+    g = torch.Generator().manual_seed(T * 7 + window)
+    q, k, v = (om.rms_norm(torch.randn(2, T, 3, 64, generator=g)).bfloat16() for _ in range(3))
+    shifted = torch.empty(v.numel() + 1, dtype=torch.bfloat16, device=dev)[1:].view(v.shape).copy_(v)
+    out = attention(q.to(dev), k.to(dev), shifted, window)
+    assert out.shape == q.shape and out.dtype == q.dtype
+    A = oc.attention_maps(*(t.double().transpose(1, 2) for t in (q, k)), window)
+    vd = v.double().transpose(1, 2)
+    err = (out.cpu().double().transpose(1, 2) - A @ vd).abs()
+    assert (err <= 2.0 ** -7 * (A @ vd.abs()) + 1e-5).all()
