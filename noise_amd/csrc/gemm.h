@@ -605,9 +605,9 @@ __global__ __launch_bounds__(256) void epi_rows_kernel(const bf16_t* __restrict_
 
 template <class S, class Epi>
 static inline hipError_t launch_gemm(const bf16_t* A, int64_t lda, const bf16_t* B, int64_t ldb, int M, int N, int K,
-                                     const Epi& epi, hipStream_t stream) {
+                                     const Epi& epi, hipStream_t stream, int splits = 1) {
   if (S::kShort && K % (2 * S::BK)) return hipErrorInvalidValue;
-  dim3 grid((N + S::BN - 1) / S::BN, (M + S::BM - 1) / S::BM);
+  dim3 grid((N + S::BN - 1) / S::BN, (M + S::BM - 1) / S::BM, splits);  // splits: the epilogue's own (blockIdx.z)
   hipLaunchKernelGGL((gemm_nt_kernel<S, Epi>), grid, dim3(S::kThreads), S::kLdsBytes, stream, A, lda, B, ldb, M, N,
                      K, epi);
   return hipGetLastError();

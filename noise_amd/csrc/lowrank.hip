@@ -15,6 +15,7 @@
 //    Both use the same rounded c, u and a; they differ only in the fp32 summation order.
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "gemm.h"
@@ -124,7 +125,8 @@ constexpr int kMemberTile = 32;  // members per MFMA tile (the N of v_mfma_f32_3
 constexpr int kURows = 128;      // rows per workgroup of shared_u_kernel (4 waves of 32)
 
 // Per member (mp workgroups; members m .. mp - 1 are zero padding): bt = bf16(b_i) [mp, in]; the bf16-rounded a_i as
-// fp32 both member-major (am [mp, out]) and column-major (at [out, mp]); asq[i] = sum_c a_i[c]^2.
+// fp32, member-major (am [mp, out], the per-element form) or column-major (at [out, mp], the expansion), the other NULL;
+// asq[i] = sum_c a_i[c]^2.
 __global__ __launch_bounds__(256) void shared_prep_kernel(const float* __restrict__ noise, int64_t stride,
                                                           int64_t a_off, int64_t b_off, int m, int mp, int in, int out,
                                                           bf16_t* __restrict__ bt, float* __restrict__ am,
@@ -137,8 +139,8 @@ __global__ __launch_bounds__(256) void shared_prep_kernel(const float* __restric
   float s = 0.f;
   for (int c = threadIdx.x; c < out; c += 256) {
     const float v = live ? bf16_to_f32(f32_to_bf16(a[c])) : 0.f;
-    am[(int64_t)i * out + c] = v;
-    at[(int64_t)c * mp + i] = v;
+    if (am) am[(int64_t)i * out + c] = v;
+    if (at) at[(int64_t)c * mp + i] = v;
     s = fmaf(v, v, s);
   }
   for (int c = threadIdx.x; c < in; c += 256) bt[(int64_t)i * in + c] = live ? f32_to_bf16(b[c]) : (bf16_t)0;
@@ -149,66 +151,75 @@ __global__ __launch_bounds__(256) void shared_prep_kernel(const float* __restric
 }
 
 // u[i, r] = bf16(x[r] . bt[i]) for every (padded) member i and row r (bf16 [mp, T]), and usq[blk, i] = sum of u[i, r]^2
-// over the workgroup's 128 rows. A wave computes 32 rows x one member tile at a time with v_mfma_f32_32x32x16_bf16,
-// its operands straight from memory: lane l reads row (or member) l % 32 at k = 8 (l / 32) .. of each 16-deep step.
+// over the workgroup's 128 rows. A wave computes 32 rows x one member tile with v_mfma_f32_32x32x16_bf16, its operands
+// straight from memory: lane l reads row (or member) l % 32 at k = 8 (l / 32) .. of each 16-deep step. Few rows are
+// bound by the latency of those reads, so a member tile has a workgroup of its own and kUDepth steps' loads are in flight
+// together (us of the expansion with the member tiles in turn and two steps in flight / here, 64 members x 512 -> 2048:
+// 2048 rows 42 / 34; 32768 rows, this kernel alone, 18 / 18).
+constexpr int kUDepth = 8;
 __global__ __launch_bounds__(256) void shared_u_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ bt,
                                                        int T, int in, int mp, bf16_t* __restrict__ u,
                                                        float* __restrict__ usq) {
   __shared__ float red[4][kMemberTile];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 5, l32 = lane & 31;
-  const int r0 = blockIdx.x * kURows + wave * 32;
+  const int r0 = blockIdx.x * kURows + wave * 32, mt = blockIdx.y;
   const bf16_t* xr = x + (int64_t)(r0 + l32) * in + 8 * g;
-  for (int mt = 0; mt < mp / kMemberTile; ++mt) {
-    const bf16_t* br = bt + (int64_t)(mt * kMemberTile + l32) * in + 8 * g;
-    f32x16 e = {};
-    for (int k = 0; k < in; k += 32) {  // in % 32 == 0
-      e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(xr + k), *(const bf16x8*)(br + k), e, 0, 0, 0);
-      e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(xr + k + 16), *(const bf16x8*)(br + k + 16), e, 0,
-                                                  0, 0);
-    }
-    // register r: row r0 + (r / 4) 8 + 4 g + r % 4, member mt 32 + l32
-    bf16_t* ur = u + (int64_t)(mt * kMemberTile + l32) * T + r0 + 4 * g;
-    float sq = 0.f;
+  const bf16_t* br = bt + (int64_t)(mt * kMemberTile + l32) * in + 8 * g;
+  f32x16 e = {};
+  int k = 0;
+  for (; k + 16 * kUDepth <= in; k += 16 * kUDepth) {
+    bf16x8 xf[kUDepth], bf[kUDepth];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t p0 = pack_bf16x2(e[4 * q], e[4 * q + 1]), p1 = pack_bf16x2(e[4 * q + 2], e[4 * q + 3]);
-      *(u32x2*)(ur + 8 * q) = u32x2{p0, p1};
-      sq = fmaf(bf16_lo(p0), bf16_lo(p0), sq);
-      sq = fmaf(bf16_hi(p0), bf16_hi(p0), sq);
-      sq = fmaf(bf16_lo(p1), bf16_lo(p1), sq);
-      sq = fmaf(bf16_hi(p1), bf16_hi(p1), sq);
+    for (int d = 0; d < kUDepth; ++d) {
+      xf[d] = *(const bf16x8*)(xr + k + 16 * d);
+      bf[d] = *(const bf16x8*)(br + k + 16 * d);
     }
-    sq += lane_xor32(sq, lane);  // lanes l and l ^ 32 hold the same member's two halves of the 32 rows
-    if (g == 0) red[wave][l32] = sq;
-    __syncthreads();
-    if (threadIdx.x < kMemberTile) {
-      const int t = threadIdx.x;
-      usq[(int64_t)blockIdx.x * mp + mt * kMemberTile + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-    }
-    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < kUDepth; ++d) e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[d], bf[d], e, 0, 0, 0);
+  }
+  for (; k < in; k += 16)  // in % 32 == 0
+    e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(xr + k), *(const bf16x8*)(br + k), e, 0, 0, 0);
+  // register r: row r0 + (r / 4) 8 + 4 g + r % 4, member mt 32 + l32
+  bf16_t* ur = u + (int64_t)(mt * kMemberTile + l32) * T + r0 + 4 * g;
+  float sq = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t p0 = pack_bf16x2(e[4 * q], e[4 * q + 1]), p1 = pack_bf16x2(e[4 * q + 2], e[4 * q + 3]);
+    *(u32x2*)(ur + 8 * q) = u32x2{p0, p1};
+    sq = fmaf(bf16_lo(p0), bf16_lo(p0), sq);
+    sq = fmaf(bf16_hi(p0), bf16_hi(p0), sq);
+    sq = fmaf(bf16_lo(p1), bf16_lo(p1), sq);
+    sq = fmaf(bf16_hi(p1), bf16_hi(p1), sq);
+  }
+  sq += lane_xor32(sq, lane);  // lanes l and l ^ 32 hold the same member's two halves of the 32 rows
+  if (g == 0) red[wave][l32] = sq;
+  __syncthreads();
+  if (threadIdx.x < kMemberTile) {
+    const int t = threadIdx.x;
+    usq[(int64_t)blockIdx.x * mp + mt * kMemberTile + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
   }
 }
 
-// The 256 x 256 tile of 4 waves of 128 x 128 that both shared-x epilogues take: 64-deep K steps in two LDS stages
-// when `in` allows (config 2, alternating builds on one box: the expansion kernel 0.100 against 0.102 ms, the
-// per-element one 0.513 against 0.524), 32-deep steps in four otherwise.
+// The 256 x 256 tile of 4 waves of 128 x 128: 64-deep K steps in two LDS stages when `in` allows (config 2,
+// alternating builds on one box: the expansion kernel 0.100 against 0.102 ms), 32-deep steps in four otherwise.
 using LTile = GemmShape<256, 256, 32, 2, 2>;
 using LTile64 = GemmShape<256, 256, 64, 2, 2, 2>;
-// The staged epilogues (per-member x, the plain linear).
 using LinTile = GemmShape<128, 256, 32, 2, 2, 3, 2>;  // two workgroups per CU
-using WideTile = GemmShape<256, 256, 64, 4, 2, 2>;    // 8 waves of 64 x 128
+using WideTile = GemmShape<256, 256, 64, 4, 2, 2>;    // 8 waves of 64 x 128 (per-member x)
 
+template <class S, class Epi>
+static hipError_t launch_shared_tile(const uint16_t* x, const uint16_t* w, int64_t T, int64_t in, int64_t out,
+                                     const Epi& epi, hipStream_t stream, int splits) {
+  const hipError_t e = prepare_gemm<S, Epi>();
+  if (e != hipSuccess) return e;
+  return launch_gemm<S>((const bf16_t*)x, in, (const bf16_t*)w, in, (int)T, (int)out, (int)in, epi, stream, splits);
+}
 template <class Epi>
 static hipError_t launch_shared_gemm(const uint16_t* x, const uint16_t* w, int64_t T, int64_t in, int64_t out,
-                                     const Epi& epi, hipStream_t stream) {
-  if (in % LTile64::BK == 0) {
-    const hipError_t e = prepare_gemm<LTile64, Epi>();
-    if (e != hipSuccess) return e;
-    return launch_gemm<LTile64>((const bf16_t*)x, in, (const bf16_t*)w, in, (int)T, (int)out, (int)in, epi, stream);
-  }
-  const hipError_t e = prepare_gemm<LTile, Epi>();
-  if (e != hipSuccess) return e;
-  return launch_gemm<LTile>((const bf16_t*)x, in, (const bf16_t*)w, in, (int)T, (int)out, (int)in, epi, stream);
+                                     const Epi& epi, hipStream_t stream, bool half, int splits) {
+  if (half) return launch_shared_tile<LinTile>(x, w, T, in, out, epi, stream, splits);
+  if (in % LTile64::BK == 0) return launch_shared_tile<LTile64>(x, w, T, in, out, epi, stream, splits);
+  return launch_shared_tile<LTile>(x, w, T, in, out, epi, stream, splits);
 }
 
 // The expansion: per tile, c2[tile] = sum of c^2 over the rounded tile, and cross[tile, i] = sum_c a_i[c] E_i[c] with
@@ -224,7 +235,7 @@ struct EpiSharedExpansion {
   template <class S>
   __device__ __forceinline__ void acc_epilogue(f32x16 (&acc)[S::TM][S::TN], unsigned char* smem, int m0, int n0,
                                                int m_tile, int n_tile, int wave, int wm, int wn, int lane) const {
-    static_assert(S::TM == 4 && S::TN == 4 && S::kWaves == 4, "a 256 x 256 tile of 4 waves of 128 x 128");
+    static_assert(S::kWaves == 4, "4 waves");
     constexpr int kLd = 17;  // padded lane stride of the partials in LDS
     float* red = (float*)smem;                    // [4 waves][64 lanes][kLd]
     float* red_c2 = red + S::kWaves * 64 * kLd;   // [4 waves]
@@ -305,7 +316,7 @@ struct EpiSharedExpansion {
 };
 
 // Per element: y = c + k_i[r] a_i[c] with k_i = s_i u_i (fp32), ss[tile, i] = sum of y^2 over the tile; optional y
-// store [m, T, out]. Members go in chunks of 64, whose k values are staged in LDS ([64][256 rows] fp32).
+// store [m, T, out]. Members go in chunks of 64, whose k values are staged in LDS ([64][BM rows] fp32).
 template <bool kStoreY>
 struct EpiSharedDirect {
   static constexpr bool kAccEpilogue = true;
@@ -314,14 +325,14 @@ struct EpiSharedDirect {
   const float* sign;   // [m]
   float* ss;           // [tiles, m]
   float* y;            // [m, T, out] when kStoreY
-  int T, m, out;
+  int T, m, out, per;  // per: members of a workgroup, blockIdx.z's of them
 
   template <class S>
   __device__ __forceinline__ void acc_epilogue(f32x16 (&acc)[S::TM][S::TN], unsigned char* smem, int m0, int n0,
                                                int m_tile, int n_tile, int wave, int wm, int wn, int lane) const {
-    static_assert(S::TM == 4 && S::TN == 4 && S::kWaves == 4 && S::BM == 256, "a 256 x 256 tile of 4 waves");
     constexpr int kChunk = 64;
-    float* ks = (float*)smem;                // [kChunk][256]
+    static_assert(S::kWaves == 4 && S::TN <= 4 && (S::BM + 4) * kChunk * 4 <= S::kLdsBytes, "4 waves; k and red fit");
+    float* ks = (float*)smem;                // [kChunk][BM]
     float* red = ks + kChunk * S::BM;        // [4 waves][kChunk]
     const int g = lane >> 5, l32 = lane & 31;
     const int tile = m_tile * gridDim.x + n_tile;
@@ -333,8 +344,9 @@ struct EpiSharedDirect {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = bf16_to_f32(f32_to_bf16(acc[i][j][r]));
 
-    for (int c0 = 0; c0 < m; c0 += kChunk) {
-      const int nm = min(kChunk, m - c0);
+    const int c_end = min(m, ((int)blockIdx.z + 1) * per);
+    for (int c0 = blockIdx.z * per; c0 < c_end; c0 += kChunk) {
+      const int nm = min(kChunk, c_end - c0);
       __syncthreads();  // the previous chunk's k values and partials have been read
       for (int idx = threadIdx.x; idx < nm * S::BM; idx += S::kThreads) {
         const int i = idx / S::BM, r = idx % S::BM;
@@ -438,8 +450,8 @@ struct SharedWs {
   float* at;    // [out, mp]
   float* asq;   // [mp]
   float* usq;   // [T / 128, mp]
-  float* c2;    // [tiles]
-  float* part;  // [tiles, mp] (cross or ss)
+  float* c2;    // [256 x 256 tiles]
+  float* part;  // [256 x 256 tiles, mp] (cross or ss)
   size_t bytes;
 };
 
@@ -542,37 +554,47 @@ static int lowrank_shared_run(const uint16_t* x, int32_t mode, const uint16_t* w
   const SharedWs ws = shared_ws(workspace, m, T, in, out);
   NOISE_REQUIRE(workspace && workspace_bytes >= ws.bytes, "workspace too small: %zu bytes needed", ws.bytes);
   const int mp = (int)((m + kMemberTile - 1) / kMemberTile * kMemberTile);
-  const int tiles = (int)((T / LTile::BM) * (out / LTile::BN));
   const int ublocks = (int)(T / kURows);
   const bool direct = mode == 2 || y != nullptr;
+  // Half tiles, two workgroups per CU. The per-element form is bound by its VALU passes over the members, and two waves
+  // per SIMD cover each other's latencies (us, 256 x 256 / 128 x 256 tiles, 64 members, 512 -> 2048: 8192 rows 151 / 110,
+  // 32768 rows 542 / 356). The expansion does twice the work per member on half tiles, so it takes them only while they
+  // are at most one per CU (64 members, 512 -> 2048: 4096 rows 51.5 / 44.5, 6144 rows 53.4 / 57.7, 32768 rows 127 / 132).
+  // Their partials are twice as many, and go where the other form's copy of a_i would be (room for 32,768 rows).
+  const int whole = (int)((T / LTile::BM) * (out / LTile::BN));
+  const bool half = direct ? T <= 32768 : whole <= 128;
+  const int tiles = half ? 2 * whole : whole;
+  float* part = !half ? ws.part : direct ? ws.at : ws.am;
+  float* c2 = half ? ws.part : ws.c2;
+  // The per-element form's members are split over workgroups that repeat a tile's product, up to one per CU (us, before /
+  // with the y stored: 24 members x 512 rows, 512 -> 2048: 115 / 49, 48 x 1024, 2048 -> 512: 270 / 93; up to two per CU
+  // 55 and 122).
+  const int64_t splits = direct ? std::min<int64_t>(m, std::max(256 / tiles, 1)) : 1;
+  const int per = (int)((m + splits - 1) / splits);
   {
     NoiseTimer tm(timed ? kTimeLowrankPre : -1, stream);
     hipLaunchKernelGGL(shared_prep_kernel, dim3(mp), dim3(256), 0, stream, noise, noise_stride, a_off, b_off, (int)m,
-                       mp, (int)in, (int)out, ws.bt, ws.am, ws.at, ws.asq);
+                       mp, (int)in, (int)out, ws.bt, direct ? ws.am : nullptr,
+                       direct ? nullptr : ws.at, ws.asq);
     NOISE_LAUNCH_CHECK();
-    hipLaunchKernelGGL(shared_u_kernel, dim3(ublocks), dim3(256), 0, stream, (const bf16_t*)x, ws.bt, (int)T, (int)in,
-                       mp, ws.u, ws.usq);
+    hipLaunchKernelGGL(shared_u_kernel, dim3(ublocks, mp / kMemberTile), dim3(256), 0, stream, (const bf16_t*)x,
+                       ws.bt, (int)T, (int)in, mp, ws.u, ws.usq);
     NOISE_LAUNCH_CHECK();
   }
   if (direct) {
-    if (y) {
-      EpiSharedDirect<true> epi{ws.u, ws.am, sign, ws.part, y, (int)T, (int)m, (int)out};
-      NoiseTimer tm(timed ? kTimeLowrank : -1, stream);
-      NOISE_CHECK_HIP(launch_shared_gemm(x, w, T, in, out, epi, stream));
-    } else {
-      EpiSharedDirect<false> epi{ws.u, ws.am, sign, ws.part, nullptr, (int)T, (int)m, (int)out};
-      NoiseTimer tm(timed ? kTimeLowrank : -1, stream);
-      NOISE_CHECK_HIP(launch_shared_gemm(x, w, T, in, out, epi, stream));
-    }
-  } else {
-    EpiSharedExpansion epi{ws.u, ws.at, ws.c2, ws.part, (int)T, mp};
     NoiseTimer tm(timed ? kTimeLowrank : -1, stream);
-    NOISE_CHECK_HIP(launch_shared_gemm(x, w, T, in, out, epi, stream));
+    auto launch = [&](auto epi) { return launch_shared_gemm(x, w, T, in, out, epi, stream, half, (int)splits); };
+    if (y) NOISE_CHECK_HIP(launch(EpiSharedDirect<true>{ws.u, ws.am, sign, part, y, (int)T, (int)m, (int)out, per}));
+    else NOISE_CHECK_HIP(launch(EpiSharedDirect<false>{ws.u, ws.am, sign, part, nullptr, (int)T, (int)m, (int)out, per}));
+  } else {
+    EpiSharedExpansion epi{ws.u, ws.at, c2, part, (int)T, mp};
+    NoiseTimer tm(timed ? kTimeLowrank : -1, stream);
+    NOISE_CHECK_HIP(launch_shared_gemm(x, w, T, in, out, epi, stream, half, 1));
   }
   if (sumsq) {
     NoiseTimer tm(timed ? kTimeLowrankPost : -1, stream);
-    hipLaunchKernelGGL(shared_finish_kernel, dim3((unsigned)m), dim3(256), 0, stream, ws.c2, ws.part, ws.usq, ws.asq,
-                       direct ? ws.part : nullptr, sign, tiles, ublocks, mp, (int)m, sumsq);
+    hipLaunchKernelGGL(shared_finish_kernel, dim3((unsigned)m), dim3(256), 0, stream, c2, part, ws.usq, ws.asq,
+                       direct ? part : nullptr, sign, tiles, ublocks, mp, (int)m, sumsq);
     NOISE_LAUNCH_CHECK();
   }
   return NOISE_OK;

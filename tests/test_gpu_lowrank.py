@@ -131,3 +131,30 @@ def test_per_member_lowrank_over_its_tiles(dev, m, T, n_in, n_out):
         bound = 2.0 ** -8 * (c.abs() + 0.5 * u.abs()[:, None] * ai.abs()) \
             + 2.0 ** -20 * (xi.abs() @ w.double().abs().t() + 0.5 * (xi.abs() @ bi.abs())[:, None] * ai.abs())
         assert ((y[i].double() - want).abs() <= bound).all(), i
+
+
+@pytest.mark.parametrize('T,n_in,n_out,m', [
+    (256, 32, 256, 1),      # the smallest; one member, so one split
+    (512, 64, 512, 130),    # a split of several members; y too
+    (8192, 64, 512, 130),   # two splits of 65 members: more than one LDS chunk of 64
+    (32768, 32, 256, 3),    # the largest on half tiles, in either form
+    (33024, 32, 256, 3),    # 256 rows more: whole tiles
+    (16896, 96, 512, 5),    # the expansion on whole tiles, the per-element form on half ones
+])
+def test_shared_tiles_and_member_splits(dev, T, n_in, n_out, m):
+    """Sums of squares on either side of the shared-x launches' rules against float64 of the bf16 operands, to the 1e-4 of
+    this file (ties of the bf16 roundings); the stored y, where it is small, against its own sums."""
+    from noise_amd.population import lowrank, lowrank_sumsq
+    print(f'lowrank shared T={T} in={n_in} out={n_out} m={m}', flush=True)
+    x, W, rows, a_off, b_off, a, b = (t.to(dev) if torch.is_tensor(t) else t for t in _inputs(T, n_in, n_out, m, seed=T + m))
+    sign = torch.where(torch.arange(m, device=dev) % 2 == 0, 0.05, -0.05).float()
+    c = (x.double() @ W.double().t()).bfloat16().double()
+    u = (x.double() @ b.bfloat16().double().t()).bfloat16().double()
+    ab = a.bfloat16().double()
+    want = torch.stack([((c + float(sign[i]) * u[:, i:i + 1] * ab[i]) ** 2).sum() for i in range(m)])
+    for mode in ('expansion', 'direct'):
+        got = lowrank_sumsq(x, W, rows, a_off, b_off, sign, mode=mode).double()
+        assert ((got - want).abs() / want).max().item() < 1e-4, mode
+    if T <= 512:
+        y = lowrank(x, W, a.contiguous(), b.contiguous(), sign).double()
+        assert (((y * y).sum((1, 2)) - want).abs() / want).max().item() < 1e-4
