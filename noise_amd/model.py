@@ -160,7 +160,8 @@ def _scan(model):
             if p is not None:
                 key.append((p.data_ptr(), p._version))
         todo.extend(c for c in m._modules.values() if c is not None)
-    key += [(b.data_ptr(), b._version) for b in (model.cos, model.sin)]
+    # buffers moved under inference_mode (parameters keep their own tensors there) have no version counter
+    key += [(b.data_ptr(), 0 if b.is_inference() else b._version) for b in (model.cos, model.sin)]
     return hooked, tuple(key)
 
 

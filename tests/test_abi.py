@@ -134,6 +134,18 @@ def test_state_dict_keys_match_reference_order():
     assert list(model.state_dict().keys()) == [n for n, _ in order]
 
 
+def test_packed_key_reads_tables_moved_under_inference_mode():
+    """Buffers that a program moved under inference_mode have no version counter; the packed operands' key must not ask
+    for it, and still changes with their storage."""
+    from noise_amd.model import GPT, GPTConfig, _scan
+    model = GPT(GPTConfig(n_layer=1, sequence_len=128))
+    hooked, key = _scan(model)
+    with torch.inference_mode():
+        model.cos, model.sin = model.cos.clone(), model.sin.clone()
+    moved = _scan(model)
+    assert (hooked, moved[0]) == (False, False) and moved[1] != key and moved == _scan(model)
+
+
 def test_eggroll_member_layout_matches_oracle():
     from noise_amd.model import GPT, GPTConfig
     from noise_amd.population import Eggroll
