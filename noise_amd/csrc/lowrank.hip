@@ -150,12 +150,38 @@ __global__ __launch_bounds__(256) void shared_prep_kernel(const float* __restric
   if (threadIdx.x == 0) asq[i] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// A wave's 32 rows x 32 members of u, from the MFMA's accumulator, and its workgroup's sums of squares.
+__device__ __forceinline__ void shared_u_store(const f32x16& e, bf16_t* __restrict__ u, float* __restrict__ usq, int T,
+                                               int mp, int r0, int m0, int block, int wave, int lane,
+                                               float (*red)[kMemberTile]) {
+  const int g = lane >> 5, l32 = lane & 31;
+  // register r: row r0 + (r / 4) 8 + 4 g + r % 4, member m0 + l32
+  bf16_t* ur = u + (int64_t)(m0 + l32) * T + r0 + 4 * g;
+  float sq = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t p0 = pack_bf16x2(e[4 * q], e[4 * q + 1]), p1 = pack_bf16x2(e[4 * q + 2], e[4 * q + 3]);
+    *(u32x2*)(ur + 8 * q) = u32x2{p0, p1};
+    sq = fmaf(bf16_lo(p0), bf16_lo(p0), sq);
+    sq = fmaf(bf16_hi(p0), bf16_hi(p0), sq);
+    sq = fmaf(bf16_lo(p1), bf16_lo(p1), sq);
+    sq = fmaf(bf16_hi(p1), bf16_hi(p1), sq);
+  }
+  sq += lane_xor32(sq, lane);  // lanes l and l ^ 32 hold the same member's two halves of the 32 rows
+  if (g == 0) red[wave][l32] = sq;
+  __syncthreads();
+  if (threadIdx.x < kMemberTile) {
+    const int t = threadIdx.x;
+    usq[(int64_t)block * mp + m0 + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+  }
+}
+
 // u[i, r] = bf16(x[r] . bt[i]) for every (padded) member i and row r (bf16 [mp, T]), and usq[blk, i] = sum of u[i, r]^2
 // over the workgroup's 128 rows. A wave computes 32 rows x one member tile with v_mfma_f32_32x32x16_bf16, its operands
 // straight from memory: lane l reads row (or member) l % 32 at k = 8 (l / 32) .. of each 16-deep step. Few rows are
 // bound by the latency of those reads, so a member tile has a workgroup of its own and kUDepth steps' loads are in flight
-// together (us of the expansion with the member tiles in turn and two steps in flight / here, 64 members x 512 -> 2048:
-// 2048 rows 42 / 34; 32768 rows, this kernel alone, 18 / 18).
+// together. For the widths that EpiSharedU's GEMM does not take (us of the expansion with the member tiles in turn and two
+// steps in flight / here, 64 members x 512 -> 2048: 2048 rows 42 / 34; 32768 rows, this kernel alone, 18 / 18).
 constexpr int kUDepth = 8;
 __global__ __launch_bounds__(256) void shared_u_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ bt,
                                                        int T, int in, int mp, bf16_t* __restrict__ u,
@@ -179,26 +205,27 @@ __global__ __launch_bounds__(256) void shared_u_kernel(const bf16_t* __restrict_
   }
   for (; k < in; k += 16)  // in % 32 == 0
     e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(xr + k), *(const bf16x8*)(br + k), e, 0, 0, 0);
-  // register r: row r0 + (r / 4) 8 + 4 g + r % 4, member mt 32 + l32
-  bf16_t* ur = u + (int64_t)(mt * kMemberTile + l32) * T + r0 + 4 * g;
-  float sq = 0.f;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t p0 = pack_bf16x2(e[4 * q], e[4 * q + 1]), p1 = pack_bf16x2(e[4 * q + 2], e[4 * q + 3]);
-    *(u32x2*)(ur + 8 * q) = u32x2{p0, p1};
-    sq = fmaf(bf16_lo(p0), bf16_lo(p0), sq);
-    sq = fmaf(bf16_hi(p0), bf16_hi(p0), sq);
-    sq = fmaf(bf16_lo(p1), bf16_lo(p1), sq);
-    sq = fmaf(bf16_hi(p1), bf16_hi(p1), sq);
-  }
-  sq += lane_xor32(sq, lane);  // lanes l and l ^ 32 hold the same member's two halves of the 32 rows
-  if (g == 0) red[wave][l32] = sq;
-  __syncthreads();
-  if (threadIdx.x < kMemberTile) {
-    const int t = threadIdx.x;
-    usq[(int64_t)blockIdx.x * mp + mt * kMemberTile + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-  }
+  shared_u_store(e, u, usq, T, mp, r0, mt * kMemberTile, blockIdx.x, wave, lane, red);
 }
+
+// The same as a GEMM, x and bt staged in LDS by whole lines: a direct load of 16 bytes from each of 32 rows uses a quarter
+// of every 128-byte line, and what a CU's waves have in flight is several times its L1, so the lines come from L2 about four
+// times (more loads in flight changed nothing). Same products in the same order. 64 members x 32,768 rows of 512: 18.1 us
+// from memory, 9.6 here (a read of x at 3.5 TB/s); the whole expansion, memory / here: 64 x 512, 512 -> 2048: 32.4 / 28.7,
+// 24 x 1024, 2048 -> 512: 63 / 43, 96 x 8192, 2048 -> 512: 76 / 55. It takes every width in its two K steps of 64.
+using UTile = GemmShape<kURows, kMemberTile, 64, 4, 1, 4, 2>;
+struct EpiSharedU {
+  static constexpr bool kAccEpilogue = true;
+  bf16_t* u;   // [mp, T]
+  float* usq;  // [T / 128, mp]
+  int T, mp;
+  template <class S>
+  __device__ __forceinline__ void acc_epilogue(f32x16 (&acc)[S::TM][S::TN], unsigned char* smem, int m0, int n0,
+                                               int m_tile, int n_tile, int wave, int wm, int wn, int lane) const {
+    static_assert(S::BM == kURows && S::BN == kMemberTile && S::kWaves == 4, "a wave's tile is 32 rows x the member tile");
+    shared_u_store(acc[0][0], u, usq, T, mp, m0 + wm * 32, n0, m_tile, wave, lane, (float (*)[kMemberTile])smem);
+  }
+};
 
 // The 256 x 256 tile of 4 waves of 128 x 128: 64-deep K steps in two LDS stages when `in` allows (config 2,
 // alternating builds on one box: the expansion kernel 0.100 against 0.102 ms), 32-deep steps in four otherwise.
@@ -577,9 +604,15 @@ static int lowrank_shared_run(const uint16_t* x, int32_t mode, const uint16_t* w
                        mp, (int)in, (int)out, ws.bt, direct ? ws.am : nullptr,
                        direct ? nullptr : ws.at, ws.asq);
     NOISE_LAUNCH_CHECK();
-    hipLaunchKernelGGL(shared_u_kernel, dim3(ublocks, mp / kMemberTile), dim3(256), 0, stream, (const bf16_t*)x,
-                       ws.bt, (int)T, (int)in, mp, ws.u, ws.usq);
-    NOISE_LAUNCH_CHECK();
+    if (in % (2 * UTile::BK) == 0 && ublocks <= 65535) { // the GEMM's K steps and grid
+      const EpiSharedU epi{ws.u, ws.usq, (int)T, mp};
+      NOISE_CHECK_HIP((prepare_gemm<UTile, EpiSharedU>()));
+      NOISE_CHECK_HIP(launch_gemm<UTile>((const bf16_t*)x, in, ws.bt, in, (int)T, mp, (int)in, epi, stream));
+    } else {
+      hipLaunchKernelGGL(shared_u_kernel, dim3(ublocks, mp / kMemberTile), dim3(256), 0, stream, (const bf16_t*)x,
+                         ws.bt, (int)T, (int)in, mp, ws.u, ws.usq);
+      NOISE_LAUNCH_CHECK();
+    }
   }
   if (direct) {
     NoiseTimer tm(timed ? kTimeLowrank : -1, stream);

@@ -158,3 +158,26 @@ def test_shared_tiles_and_member_splits(dev, T, n_in, n_out, m):
     if T <= 512:
         y = lowrank(x, W, a.contiguous(), b.contiguous(), sign).double()
         assert (((y * y).sum((1, 2)) - want).abs() / want).max().item() < 1e-4
+
+
+@pytest.mark.parametrize('T,n_in,n_out,m', [
+    (256, 128, 256, 1),    # the smallest: two K steps, fewer than the stages; one member of its tile of 32
+    (512, 256, 256, 33),   # as many steps as stages; a second tile of one member
+    (768, 640, 512, 96),   # three member tiles
+    (1024, 2048, 256, 40),
+])
+def test_member_dots_are_the_same_bits_staged_or_from_memory(dev, T, n_in, n_out, m):
+    """x . b of a width in 128-column steps runs as a GEMM through LDS, of other widths straight from memory: 32 columns of
+    zeros more change the route and add exact zeros to every product, so every sum of squares keeps its bits."""
+    from noise_amd.population import lowrank_sumsq
+    print(f'lowrank shared dots T={T} in={n_in} out={n_out} m={m}', flush=True)
+    x, W, rows, a_off, b_off, a, b = (t.to(dev) if torch.is_tensor(t) else t for t in _inputs(T, n_in, n_out, m, seed=T + m))
+    sign = torch.where(torch.arange(m, device=dev) % 2 == 0, 0.5, -0.5).float()
+    wide = [torch.nn.functional.pad(t, (0, 32)).contiguous() for t in (x, W, b)]
+    wide_rows = torch.cat([a, wide[2]], 1).contiguous()
+    u = x.double() @ b.bfloat16().double().t()
+    assert u.abs().mean().item() > 1  # the members' terms are no small part of the sums
+    for mode in ('expansion', 'direct'):
+        got = lowrank_sumsq(x, W, rows, a_off, b_off, sign, mode=mode)
+        want = lowrank_sumsq(wide[0], wide[1], wide_rows, 0, n_out, sign, mode=mode)
+        assert torch.isfinite(got).all() and torch.equal(got, want), mode
