@@ -482,8 +482,8 @@ def bench_head_error(dev, iters=3):
     jittered = draws * b * t * 256
     return dict(ms=round(ms, 3), draws=draws, token_rows=b * t, vocab=V, finite=bool(torch.isfinite(err).all()),
                 jittered_logits_per_s=round(jittered / (ms * 1e-3), 1),
-                note='per call: 9,216 draws x 16,384 token rows x one 256-column slab, the jitter regenerated '
-                     'twice from the counter stream (loss, then error), never stored')
+                note='per call: 9,216 draws x 16,384 token rows x one 256-column slab, the jitter made '
+                     'once per draw from the counter stream, never stored')
 
 
 def bench_dust_direct(dev, model, iters=2):

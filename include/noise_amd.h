@@ -199,7 +199,7 @@ int noise_fitness(const float* losses, int64_t members, int64_t pairs, float* fi
 int noise_outer_grad(const float* rows, int64_t stride, int64_t a_off, int64_t b_off, const float* weight,
                      int64_t pairs, int64_t out, int64_t in, float scale, int32_t accumulate, float* grad, void* stream);
 
-/* noise_outer_grad for n matrices in one launch (fp32 MFMA, 128 x 128 output tiles; each matrix j as noise_outer_grad
+/* noise_outer_grad for n matrices in one launch (fp32 MFMA; each matrix j as noise_outer_grad
  * with a_off[j], b_off[j] >= 0, out[j], in[j] and grads[j], a host array of device pointers). The per-parameter loop
  * of the update becomes one grid that fills the GPU even where single matrices are small (512 x 512).
  * Replaces: archive/10M/train/val/eggroll.py:155-163 (the loop over parameters and chunks of directions). */
